@@ -183,6 +183,7 @@ struct ctl_batch {
     std::vector<int> K, SS, lanes;
     KParams* d_desc = nullptr;
     uint32_t* d_rep_next = nullptr;            // per-model replica counters
+    uint32_t* h_done = nullptr;                // per-class done counters (pinned host memory)
     std::vector<BClass> classes;
     int verbose = 0;
     std::vector<void*> allocs;
@@ -225,6 +226,8 @@ int bupload(ctl_batch* b, T** p, const T* src, size_t count) {
 void brelease(ctl_batch* b) {
     for (void* q : b->allocs) (void)hipFree(q);
     b->allocs.clear();
+    if (b->h_done) (void)hipHostFree(b->h_done);
+    b->h_done = nullptr;
     for (BClass& c : b->classes) {
         if (c.ev0) (void)hipEventDestroy(c.ev0);
         if (c.ev1) (void)hipEventDestroy(c.ev1);
@@ -403,6 +406,8 @@ int ctl_batch_create_lanes(const ctl_model* const* models, const int64_t* replic
         if (!c.models.empty()) b->classes.push_back(c);
     }
     if ((rc = balloc(b, &b->d_rep_next, nmodels))) return bail(rc);
+    if ((e = hipHostMalloc((void**)&b->h_done, sizeof(uint32_t) * b->classes.size(), hipHostMallocDefault)) != hipSuccess)
+        return bail(bhip(e, "hipHostMalloc"));
     std::vector<int> cls(nmodels, -1);
     for (size_t k = 0; k < b->classes.size(); ++k) {
         BClass& c = b->classes[k];
@@ -621,13 +626,18 @@ int ctl_batch_run(ctl_batch* b) {
     BHIP(hipMemset(b->d_rep_next, 0, sizeof(uint32_t) * b->nmodels), "memset");
     ctl_stats& S = b->stats;
     S.launches = 0;
-    // the classes run concurrently: each round launches every unfinished
-    // class on its own stream, then waits for all of them
+    // The classes run concurrently: each round launches every unfinished
+    // class on its own stream, then waits for all of them.  The done counters
+    // come back in pinned memory: a copy to pageable memory returns only when
+    // it is done, so the second class's kernel would start after the first's
+    // end (64 uneven models in six classes: the kernels of 18 to 165 ms one
+    // after the other, 430 ms).  Widest class first: it holds the largest
+    // models, whose chains of steps are the longest.
     const auto k0 = std::chrono::steady_clock::now();
-    std::vector<uint32_t> done(b->classes.size(), 0);
+    volatile uint32_t* done = b->h_done;
     for (;;) {
         bool any = false;
-        for (size_t k = 0; k < b->classes.size(); ++k) {
+        for (size_t k = b->classes.size(); k-- > 0;) {
             BClass& c = b->classes[k];
             if (c.finished) continue;
             any = true;
@@ -646,7 +656,7 @@ int ctl_batch_run(ctl_batch* b) {
                 }
             BHIP(hipGetLastError(), "batch kernel launch");
             BHIP(hipEventRecord(c.ev1, c.stream), "hipEventRecord");
-            BHIP(hipMemcpyAsync(&done[k], c.d_done, sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream), "hipMemcpy D2H");
+            BHIP(hipMemcpyAsync(b->h_done + k, c.d_done, sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream), "hipMemcpy D2H");
             ++S.launches;
         }
         if (!any) break;
@@ -658,7 +668,7 @@ int ctl_batch_run(ctl_batch* b) {
             if (b->verbose) {
                 float ms = 0.0f;
                 (void)hipEventElapsedTime(&ms, c.ev0, c.ev1);
-                std::fprintf(stderr, " * class G=%d launch: %u/%lld simulations done (%.3f ms)\n", c.G, done[k],
+                std::fprintf(stderr, " * class G=%d launch: %u/%lld simulations done (%.3f ms)\n", c.G, (unsigned)done[k],
                              (long long)c.total, ms);
             }
         }
