@@ -6,8 +6,9 @@
 // model, auto_lanes), and the models of one G form a class with its own
 // persistent kernel on its own stream; the classes run concurrently:
 //   G = 1      batch_kernel (below): one simulation per lane;
-//   G = 2..32  gclass_kernel<G> (ctl_gbatch.hip): 64/G groups of a wavefront
-//              run replicas of one model, the simulations' state in LDS;
+//   G = 2..32  gclass_kernel<G, W> (ctl_gbatch.hip): 64/W groups of a wavefront
+//              (W lanes each, W = G unless the class leaves the chip short of
+//              wavefronts) run replicas of one model, the state in LDS;
 //   G = 64     gbatch_kernel (ctl_gbatch.hip): one wavefront per simulation.
 // Inside a class the work is ordered by an estimated cost, largest first.
 //
@@ -156,10 +157,11 @@ using namespace ctl;
 
 // The models of a batch that run with the same lanes per simulation G form
 // a class: one persistent kernel on its own stream (G = 1: batch_kernel,
-// G = 2..32: gclass_kernel<G>, G = 64: gbatch_kernel).  The classes of a
+// G = 2..32: gclass_kernel<G, W>, G = 64: gbatch_kernel).  The classes of a
 // batch run concurrently.
 struct BClass {
     int G = 1;
+    int W = 1;                                // lanes that execute one simulation (>= G)
     std::vector<int> models;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -251,7 +253,7 @@ int auto_lanes(const ctl::Model& m) {
 }
 
 // Per-model device tables (the same compile products as a ctl_sim).
-int upload_model(ctl_batch* b, const ctl::Model& m, KParams& p, int G) {
+int upload_model(ctl_batch* b, const ctl::Model& m, KParams& p, int G, int W) {
     const int S = m.S, R = m.R;
     std::vector<uint32_t> horw(S);
     for (int i = 0; i < S; ++i) horw[i] = (uint32_t)m.hor[i] | ((uint32_t)m.hort[i] << 8);
@@ -329,7 +331,7 @@ int upload_model(ctl_batch* b, const ctl::Model& m, KParams& p, int G) {
         p.oDp = put(Dptr.data(), Dptr.size());
         p.oDe = put(Dent.data(), Dent.size());
         p.oCs = put(reinterpret_cast<const uint32_t*>(m.cs.data()), m.cs.size());
-        if (G > 1) append_group_streams(T, p, G, m, FSptr, FSent, Dent);
+        if (G > 1) append_group_streams(T, p, G, W, m, FSptr, FSent, Dent);
         uint32_t* Td;
         if ((rc = bupload(b, &Td, T.data(), T.size()))) return rc;
         p.T = Td;
@@ -400,7 +402,7 @@ int ctl_batch_create_lanes(const ctl_model* const* models, const int64_t* replic
     // classes, ascending G
     for (int G = 1; G <= 64; G *= 2) {
         BClass c;
-        c.G = G;
+        c.G = c.W = G;
         for (int i = 0; i < nmodels; ++i)
             if (lanes[i] == G) { c.models.push_back(i); c.total += replicas[i]; }
         if (!c.models.empty()) b->classes.push_back(c);
@@ -478,10 +480,23 @@ int ctl_batch_create_lanes(const ctl_model* const* models, const int64_t* replic
                 return bail(rc);
             g.iters = o->iters_per_launch > 0 ? o->iters_per_launch : 65536;
         } else {
-            const int gpw = 64 / c.G;                       // groups per wavefront (= workgroup)
+            // the widest W at which every replica of the class is resident at
+            // once, as ctl_sim_create chooses it for one model; an explicit
+            // slot count keeps W = G
+            c.W = c.G;
+            for (int w = 64; o->slots <= 0 && w > c.G && w >= 32; w /= 2) {
+                int cu = 0;
+                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&cu, ctl::gclass_kernel_fn(c.G, w), 64,
+                                                                 (size_t)(64 / w) * gwords * 4);
+                if (e == hipSuccess && (long long)prop.multiProcessorCount * cu * (64 / w) >= c.total) {
+                    c.W = w;
+                    break;
+                }
+            }
+            const int gpw = 64 / c.W;                       // groups per wavefront (= workgroup)
             c.block = 64;
             c.smem = (size_t)gpw * gwords * 4;
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ctl::gclass_kernel_fn(c.G), 64, c.smem);
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ctl::gclass_kernel_fn(c.G, c.W), 64, c.smem);
             if (e != hipSuccess || per_cu <= 0) per_cu = 1;
             long long waves = o->slots > 0 ? ((long long)o->slots + gpw - 1) / gpw
                                            : (long long)prop.multiProcessorCount * per_cu;
@@ -498,8 +513,8 @@ int ctl_batch_create_lanes(const ctl_model* const* models, const int64_t* replic
                 (rc = balloc(b, &g.t, ng)) || (rc = balloc(b, &g.cursor, ng)) || (rc = balloc(b, &g.evc, ng)) ||
                 (rc = balloc(b, &g.firings, ng)) || (rc = balloc(b, &g.ssa_steps, ng)) ||
                 (rc = balloc(b, &g.leaps, ng)) || (rc = balloc(b, &g.rejections, ng)) ||
-                (rc = balloc(b, &g.switches, ng)) || (rc = balloc(b, &g.poisson, ng * c.G)) ||
-                (rc = balloc(b, &g.gaps, ng * c.G)) || (rc = balloc(b, &g.X, ng * maxS)) ||
+                (rc = balloc(b, &g.switches, ng)) || (rc = balloc(b, &g.poisson, ng * c.W)) ||
+                (rc = balloc(b, &g.gaps, ng * c.W)) || (rc = balloc(b, &g.X, ng * maxS)) ||
                 (rc = balloc(b, &g.chunk_next, 1)))
                 return bail(rc);
             g.iters = o->iters_per_launch > 0 ? o->iters_per_launch : 65536;
@@ -516,7 +531,7 @@ int ctl_batch_create_lanes(const ctl_model* const* models, const int64_t* replic
         const ctl::Model& m = models[i]->m;
         const BClass& c = b->classes[cls[i]];
         KParams p{};
-        if ((rc = upload_model(b, m, p, lanes[i]))) return bail(rc);
+        if ((rc = upload_model(b, m, p, lanes[i], c.W))) return bail(rc);
         p.n = (int)replicas[i];
         p.x0_div = (m.x0_rows <= 1 || m.x0_rows >= p.n) ? 1 : (int)(p.n / m.x0_rows);
         p.c_div = (m.c_rows <= 1 || m.c_rows >= p.n) ? 1 : (int)(p.n / m.c_rows);
@@ -569,7 +584,7 @@ int ctl_batch_create_lanes(const ctl_model* const* models, const int64_t* replic
             g.cum = d_cum;
             g.nmodels = (int)order.size();
         } else {                               // chunks of one wavefront's worth of replicas
-            const int per = c.G == 1 ? 64 : 64 / c.G;
+            const int per = c.G == 1 ? 64 : 64 / c.W;
             std::vector<int32_t> chunks;
             for (int i : order)
                 for (int64_t r = 0; r < b->reps[i]; r += per) chunks.push_back(i);
@@ -646,14 +661,11 @@ int ctl_batch_run(ctl_batch* b) {
                 hipLaunchKernelGGL(batch_kernel, dim3(c.grid), dim3(c.block), 0, c.stream, c.bp);
             else if (c.G == 64)
                 hipLaunchKernelGGL(gbatch_kernel, dim3(c.grid), dim3(64), c.smem, c.stream, c.gp);
-            else
-                switch (c.G) {
-                    case 2: hipLaunchKernelGGL(gclass_kernel<2>, dim3(c.grid), dim3(64), c.smem, c.stream, c.cp); break;
-                    case 4: hipLaunchKernelGGL(gclass_kernel<4>, dim3(c.grid), dim3(64), c.smem, c.stream, c.cp); break;
-                    case 8: hipLaunchKernelGGL(gclass_kernel<8>, dim3(c.grid), dim3(64), c.smem, c.stream, c.cp); break;
-                    case 16: hipLaunchKernelGGL(gclass_kernel<16>, dim3(c.grid), dim3(64), c.smem, c.stream, c.cp); break;
-                    default: hipLaunchKernelGGL(gclass_kernel<32>, dim3(c.grid), dim3(64), c.smem, c.stream, c.cp); break;
-                }
+            else {
+                void* args[] = {&c.cp};
+                BHIP(hipLaunchKernel(ctl::gclass_kernel_fn(c.G, c.W), dim3(c.grid), dim3(64), args, c.smem, c.stream),
+                     "gclass_kernel launch");
+            }
             BHIP(hipGetLastError(), "batch kernel launch");
             BHIP(hipEventRecord(c.ev1, c.stream), "hipEventRecord");
             BHIP(hipMemcpyAsync(b->h_done + k, c.d_done, sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream), "hipMemcpy D2H");

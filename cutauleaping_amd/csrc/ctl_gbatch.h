@@ -46,8 +46,8 @@ static __device__ __forceinline__ KParams desc_of_b(const KParams* desc, int m) 
 
 __global__ void gbatch_kernel(GBatchParams bp);
 
-// Group batch with G = 2..32 lanes per simulation: a 64-lane wavefront holds
-// 64 / G groups that all run replicas of one model at a time (the model is
+// Group batch with G = 2..32 lanes per simulation, each executed by W >= G
+// lanes: a 64-lane wavefront holds 64 / W groups that all run replicas of one model at a time (the model is
 // wave-uniform, so its tables stay scalar loads).  The wavefront takes the
 // next chunk of the class's chunk list (chunks name models, largest work
 // first); its groups then pull replicas of that model from the model's own
@@ -73,13 +73,13 @@ struct GClassParams {
     uint32_t* leaps;
     uint32_t* rejections;
     uint32_t* switches;
-    uint64_t* poisson;          // [slot][G]
-    uint64_t* gaps;             // [slot][G]
+    uint64_t* poisson;          // [slot][W]
+    uint64_t* gaps;             // [slot][W]
     int32_t* X;                 // [slot][maxS]
 };
 
-template <int G>
+template <int G, int W>
 __global__ void gclass_kernel(GClassParams bp);
-const void* gclass_kernel_fn(int G);
+const void* gclass_kernel_fn(int G, int W);     // W = G, 32 or 64
 
 }  // namespace ctl

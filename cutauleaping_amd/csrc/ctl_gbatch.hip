@@ -37,7 +37,7 @@ __global__ __launch_bounds__(64) void gbatch_kernel(GBatchParams bp) {
     if (L.sim >= 0) {                    // resume a parked simulation
         p = desc_of_b(bp.desc, m);
         V = group_view(smem, p.S, p.R, G);
-        gzero_pad<G>(V, p.R, l);
+        gzero_pad<G, G>(V, p.R, l);
         L.t = bp.t[slot];
         L.cursor = bp.cursor[slot];
         L.evc = bp.evc[slot];
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(64) void gbatch_kernel(GBatchParams bp) {
             const uint32_t r = (uint32_t)((int64_t)q - CT_I64(bp.cum)[lo]);
             p = desc_of_b(bp.desc, m);
             V = group_view(smem, p.S, p.R, G);
-            gzero_pad<G>(V, p.R, l);
+            gzero_pad<G, G>(V, p.R, l);
             L.sim = (int)r;
             L.t = 0.0;
             L.cursor = 0;
@@ -97,14 +97,14 @@ __global__ __launch_bounds__(64) void gbatch_kernel(GBatchParams bp) {
             gsync();
         }
         if (p.force_ssa) {
-            if (L.t >= p.tmax || gssa<G>(p, L, V, l)) gfinish<G>(p, L, V, l);
+            if (L.t >= p.tmax || gssa<G, G>(p, L, V, l)) gfinish<G>(p, L, V, l);
             continue;
         }
-        const int r = gleap<G>(p, L, V, l, recip);
+        const int r = gleap<G, G>(p, L, V, l, recip);
         if (r == LEAP_DONE || r == LEAP_ABSORB) {
             gfinish<G>(p, L, V, l);
         } else if (r == LEAP_SWITCH) {
-            if (gssa<G>(p, L, V, l)) gfinish<G>(p, L, V, l);
+            if (gssa<G, G>(p, L, V, l)) gfinish<G>(p, L, V, l);
         }
     }
     if (L.sim >= 0) {                    // park
@@ -134,15 +134,15 @@ __global__ __launch_bounds__(64) void gbatch_kernel(GBatchParams bp) {
 // group of the wavefront switches (at most GBURST_WAIT iterations, or until
 // every group with a replica waits); a group without a replica idles.  Each
 // replica's trajectory depends only on its own state and streams.
-template <int G>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 8 || G == 16 || G == 32 ? 4 : 1)))
+template <int G, int W>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(gwaves(G, W))))
 void gclass_kernel(GClassParams bp) {
     extern __shared__ uint32_t smem[];
     __shared__ float recip[64];
     recip[threadIdx.x] = c_recip[threadIdx.x];
     __syncthreads();
-    const int l = (int)(threadIdx.x & (unsigned)(G - 1));
-    const int gib = (int)(threadIdx.x / G);
+    const int l = (int)(threadIdx.x & (unsigned)(W - 1));
+    const int gib = (int)(threadIdx.x / W);
     const int wave = (int)blockIdx.x;
     if (wave >= bp.nwaves) return;
     uint32_t* gbase = smem + (size_t)gib * (size_t)bp.gwords;
@@ -150,14 +150,14 @@ void gclass_kernel(GClassParams bp) {
     L.tacc = 0.0;
     L.ssa_left = 0;
     L.ssa_mode = 0;
-    L.slot = wave * (64 / G) + gib;
-    L.lg.tag = 1u + (uint32_t)l;
+    L.slot = wave * (64 / W) + gib;
+    L.lg.tag = 1u + (uint32_t)(l & (G - 1));
     int m = __builtin_amdgcn_readfirstlane(bp.wave_model[wave]);
     L.sim = m >= 0 ? bp.slot_sim[L.slot] : -1;
     if (m >= 0) {
         const KParams p = desc_of_b(bp.desc, m);
         const GView V = group_view(gbase, p.S, p.R, G);
-        gzero_pad<G>(V, p.R, l);
+        gzero_pad<G, W>(V, p.R, l);
         L.gg.k0 = L.lg.k0 = p.key0;
         L.gg.k1 = L.lg.k1 = p.key1;
         if (L.sim >= 0) {                // resume a parked replica
@@ -172,12 +172,12 @@ void gclass_kernel(GClassParams bp) {
             L.rejections = bp.rejections[s0];
             L.switches = bp.switches[s0];
             L.absorbed = 0;
-            L.poisson = bp.poisson[(size_t)s0 * G + l];
-            L.gaps = bp.gaps[(size_t)s0 * G + l];
+            L.poisson = bp.poisson[(size_t)s0 * W + l];
+            L.gaps = bp.gaps[(size_t)s0 * W + l];
             L.gg.sim = L.lg.sim = p.sim_base + (uint32_t)L.sim;
             L.gg.cb = GRNG_NONE;
             L.lg.pos = 4;
-            for (int s = l; s < p.S; s += G) V.Xb[s] = bp.X[(size_t)s0 * bp.maxS + s];
+            for (int s = l; s < p.S; s += W) V.Xb[s] = bp.X[(size_t)s0 * bp.maxS + s];
             L.crate = grates(p, L.sim);
             L.fvrow = p.nfs > 0 ? p.fv + (size_t)(L.sim / p.fv_div) * p.nfs : nullptr;
         }
@@ -193,7 +193,7 @@ void gclass_kernel(GClassParams bp) {
             if (c >= (uint32_t)bp.nchunks) break;
             m = __builtin_amdgcn_readfirstlane(CT_I32(bp.chunk_model)[c]);
             const KParams p = desc_of_b(bp.desc, m);
-            gzero_pad<G>(group_view(gbase, p.S, p.R, G), p.R, l);
+            gzero_pad<G, W>(group_view(gbase, p.S, p.R, G), p.R, l);
             L.sim = -1;
         }
         const KParams p = desc_of_b(bp.desc, m);
@@ -201,17 +201,17 @@ void gclass_kernel(GClassParams bp) {
         if (L.sim == -1) {               // a replica of the model (-2 once it has none left)
             L.gg.k0 = L.lg.k0 = p.key0;
             L.gg.k1 = L.lg.k1 = p.key1;
-            gfetch<G>(p, L, V, l);
+            gfetch<W>(p, L, V, l);
         }
         if (__ballot(L.sim >= 0) == 0) { m = -1; continue; }
         const bool active = L.sim >= 0;
         if (active) {
             if (kuse(p.force_ssa)) {
-                if (L.t >= p.tmax || gssa<G>(p, L, V, l)) gfinish<G>(p, L, V, l);
+                if (L.t >= p.tmax || gssa<G, W>(p, L, V, l)) gfinish<W>(p, L, V, l);
             } else if (!pend) {
-                const int r = gleap<G>(p, L, V, l, recip);
+                const int r = gleap<G, W>(p, L, V, l, recip);
                 if (r == LEAP_DONE || r == LEAP_ABSORB) {
-                    gfinish<G>(p, L, V, l);
+                    gfinish<W>(p, L, V, l);
                 } else if (r == LEAP_SWITCH) {
                     pend = true;
                     waited = 0;
@@ -225,19 +225,19 @@ void gclass_kernel(GClassParams bp) {
         const bool go = pm != 0 && (__popcll(pm) >= 2 || pm == lead || __ballot(pend && waited >= GBURST_WAIT) != 0);
         if (go && pend) {
             pend = false;
-            if (gssa<G>(p, L, V, l)) gfinish<G>(p, L, V, l);
+            if (gssa<G, W>(p, L, V, l)) gfinish<W>(p, L, V, l);
         }
     }
     if (m >= 0) {
         const KParams p = desc_of_b(bp.desc, m);
         const GView V = group_view(gbase, p.S, p.R, G);
-        if (pend && gssa<G>(p, L, V, l)) gfinish<G>(p, L, V, l);   // before parking
+        if (pend && gssa<G, W>(p, L, V, l)) gfinish<W>(p, L, V, l);   // before parking
         if (L.sim >= 0) {                // park
             const int s0 = L.slot;
             const int32_t* X = V.Xb + (L.xb ? p.S : 0);
-            for (int s = l; s < p.S; s += G) bp.X[(size_t)s0 * bp.maxS + s] = X[s];
-            bp.poisson[(size_t)s0 * G + l] = L.poisson;
-            bp.gaps[(size_t)s0 * G + l] = L.gaps;
+            for (int s = l; s < p.S; s += W) bp.X[(size_t)s0 * bp.maxS + s] = X[s];
+            bp.poisson[(size_t)s0 * W + l] = L.poisson;
+            bp.gaps[(size_t)s0 * W + l] = L.gaps;
             if (l == 0) {
                 bp.t[s0] = L.t;
                 bp.cursor[s0] = L.cursor;
@@ -254,19 +254,22 @@ void gclass_kernel(GClassParams bp) {
     if (threadIdx.x == 0) bp.wave_model[wave] = m;
 }
 
-template __global__ void gclass_kernel<2>(GClassParams);
-template __global__ void gclass_kernel<4>(GClassParams);
-template __global__ void gclass_kernel<8>(GClassParams);
-template __global__ void gclass_kernel<16>(GClassParams);
-template __global__ void gclass_kernel<32>(GClassParams);
+template <int G>
+static const void* gclass_fn_g(int W) {
+    if (W == G) return (const void*)gclass_kernel<G, G>;
+    if constexpr (G < 32) {
+        if (W == 32) return (const void*)gclass_kernel<G, 32>;
+    }
+    return W == 64 ? (const void*)gclass_kernel<G, 64> : nullptr;
+}
 
-const void* gclass_kernel_fn(int G) {
+const void* gclass_kernel_fn(int G, int W) {
     switch (G) {
-        case 2: return (const void*)gclass_kernel<2>;
-        case 4: return (const void*)gclass_kernel<4>;
-        case 8: return (const void*)gclass_kernel<8>;
-        case 16: return (const void*)gclass_kernel<16>;
-        case 32: return (const void*)gclass_kernel<32>;
+        case 2: return gclass_fn_g<2>(W);
+        case 4: return gclass_fn_g<4>(W);
+        case 8: return gclass_fn_g<8>(W);
+        case 16: return gclass_fn_g<16>(W);
+        case 32: return gclass_fn_g<32>(W);
     }
     return nullptr;
 }

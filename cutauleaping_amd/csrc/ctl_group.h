@@ -22,6 +22,15 @@
 // DPP row operations and lane reads and are identical in every lane of the
 // group, so the group's control flow is uniform.
 //
+// Two widths: G is the algorithm's (whose partial sums and lane streams fix a
+// trajectory's bits), W >= G the lanes that execute one simulation.  With
+// W > G, lane l stands for the algorithm's lane l mod G (W / G lanes hold the
+// same partial sums and streams); the work whose result does not depend on the
+// lane that does it -- a reaction's propensity, a species' tau' and update, a
+// queued Poisson draw, a sample, a dependent -- is spread over all W.  A run
+// whose simulations do not fill the chip takes a larger W (gwidth), down to
+// one simulation per wavefront.
+//
 // Algorithm (restated lane by lane by the oracle's group mode):
 //  * propensities and criticality per reaction as in the one-lane kernel;
 //  * a0 and every cumulative selection use the lane partial sums (each
@@ -315,10 +324,10 @@ __device__ __forceinline__ void grng_event(GRng& g, uint32_t ev) {
     g.cb = GRNG_NONE;
 }
 
-template <int G>
+template <int W>
 __device__ __forceinline__ uint32_t grng_u32(GRng& g, int l) {
     const uint32_t b = g.wc >> 2;
-    if (b - g.cb >= (uint32_t)G) {
+    if (b - g.cb >= (uint32_t)W) {
         g.cb = b;
         philox_block(b + (uint32_t)l, g.ev, g.sim, 0u, g.k0, g.k1, g.c0, g.c1, g.c2, g.c3);
     }
@@ -333,7 +342,7 @@ __device__ __forceinline__ uint32_t grng_u32(GRng& g, int l) {
     const uint32_t mine = (k & 2u) ? hi : lo;
     const int src = (int)(b - g.cb);
     g.wc += 1u;
-    return __shfl(mine, src, G);
+    return __shfl(mine, src, W);
 }
 
 struct GLane {
@@ -407,17 +416,17 @@ __device__ __forceinline__ void gfactor(uint32_t* F, int S, int s, int32_t x, ui
 
 // The whole factor table of state X; F[2S] = 1.0 is the factor of a padding
 // entry (multiplicity 0), never critical.
-template <int G>
+template <int W>
 __device__ __forceinline__ void gfactors(const KParams& p, const int32_t* X, uint32_t* F, int l) {
     const uint32_t nc = (uint32_t)p.nc;
-    for (int s = l; s < p.S; s += G) gfactor(F, p.S, s, X[s], nc);
+    for (int s = l; s < p.S; s += W) gfactor(F, p.S, s, X[s], nc);
     if (l == 0) F[2 * p.S] = 0x3f800000u;
 }
 
 // Zeroes a group's A padding (R .. Rp-1); done when the group's model is set.
-template <int G>
+template <int G, int W>
 __device__ __forceinline__ void gzero_pad(const GView& V, int R, int l) {
-    for (int j = R + l; j < group_rpad(R, G); j += G) V.A[j] = 0u;
+    for (int j = R + l; j < group_rpad(R, G); j += W) V.A[j] = 0u;
 }
 
 // Propensity of reaction j from the group's LDS state; the arithmetic of
@@ -449,6 +458,81 @@ __device__ __forceinline__ float gprop(const KParams& p, const int32_t* X, const
     return a;
 }
 
+// gprops with W > G lanes per simulation: lane l computes reactions l, l + W,
+// ..., so a round of W lanes covers W / G of the algorithm's rounds; then every
+// algorithm lane's partial sums are added from LDS in ascending round order
+// (the W / G lanes that stand for one algorithm lane do so redundantly).  The
+// propensities are the same values, the sums the same additions.
+template <int G, int W, int PFM>
+__device__ __forceinline__ void gprops_wide(const KParams& p, const int32_t* X, const uint32_t* F, const float* crate,
+                                            uint32_t* A, int l, float& P, float& PC) {
+    const int pm = pmode<PFM>(kuse(p.pfast));
+    const uint32_t nc = (uint32_t)p.nc;
+    const int a0 = l & (G - 1);
+    if (pm != 0) {
+        const uint32_t* E = p.T + p.oPRe;
+        for (int j0 = l; j0 < p.R; j0 += 4 * W) {
+            float cr[4];
+            uint32_t e0[4], e1[4], u0[4], u1[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int j = j0 + q * W;
+                cr[q] = 0.0f;
+                e0[q] = e1[q] = pm == 1 ? (uint32_t)(2 * p.S) : 0u;
+                if (j < p.R) {
+                    const uint32_t* Er = E + (2 * (j / G)) * G + a0;
+                    e0[q] = Er[0];
+                    e1[q] = Er[G];
+                    cr[q] = crate[j];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                u0[q] = pm == 1 ? F[e0[q]] : (uint32_t)X[e0[q] & 0xffffu];
+                u1[q] = pm == 1 ? F[e1[q]] : (uint32_t)X[e1[q] & 0xffffu];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int j = j0 + q * W;
+                if (j < p.R) {
+                    float a = cr[q];
+                    uint32_t cbit;
+                    if (pm == 1) {
+                        a = a * __uint_as_float(u0[q] & 0x7fffffffu);
+                        a = a * __uint_as_float(u1[q] & 0x7fffffffu);
+                        cbit = (u0[q] | u1[q]) & 0x80000000u;
+                    } else {
+                        bool c = false;
+                        gtwo(a, c, (int32_t)u0[q], e0[q] >> 16, (int32_t)u1[q], e1[q] >> 16, nc);
+                        cbit = c ? 0x80000000u : 0u;
+                    }
+                    A[j] = __float_as_uint(a) | cbit;
+                }
+            }
+        }
+    } else {
+        for (int j = l; j < p.R; j += W) {
+            bool c;
+            const float a = gprop(p, X, crate, j, c);
+            A[j] = __float_as_uint(a) | (c ? 0x80000000u : 0u);
+        }
+    }
+    gsync();
+    P = 0.0f;
+    PC = 0.0f;
+    const int nrp = group_rpad(p.R, G) / G;
+    for (int r0 = 0; r0 < nrp; r0 += 4) {              // padding adds an exact 0
+        uint32_t u[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u[i] = r0 + i < nrp ? A[a0 + (r0 + i) * G] : 0u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            P = P + aval(u[i]);
+            if (u[i] & 0x80000000u) PC = PC + aval(u[i]);
+        }
+    }
+}
+
 // Every reaction of lane l (j = l, l + G, ...) from the reactant round
 // stream: the table addresses do not depend on loaded data, so the loads of a
 // round issue together.  Writes A[j] (propensity bits | critical << 31) and
@@ -456,9 +540,13 @@ __device__ __forceinline__ float gprop(const KParams& p, const int32_t* X, const
 // With pfast the two entries of a reaction are indices into the factor table
 // F of the state (built by gfactors), so a reaction costs two multiplies:
 // the same factors in the same order as greactant, hence the same bits.
-template <int G, int PFM = 3>
+template <int G, int W, int PFM = 3>
 __device__ __forceinline__ void gprops(const KParams& p, const int32_t* X, const uint32_t* F, const float* crate,
                                        uint32_t* A, int l, float& P, float& PC) {
+    if constexpr (W > G) {
+        gprops_wide<G, W, PFM>(p, X, F, crate, A, l, P, PC);
+        return;
+    }
     const int nr = (p.R + G - 1) / G;
     P = 0.0f;
     PC = 0.0f;
@@ -614,50 +702,52 @@ __device__ __forceinline__ int gselect(const KParams& p, const uint32_t* A, floa
     return last;
 }
 
-template <int G>
+template <int W>
 __device__ __forceinline__ void gabsorb(const KParams& p, GLane& L, const int32_t* X, int l) {
     uint32_t* out = p.storage + (size_t)L.sim * p.K * p.SS;
     if (L.cursor == 0) {
-        for (int sk = l; sk < p.SS; sk += G) out[sk] = (uint32_t)X[p.T[p.oCs + sk]];
+        for (int sk = l; sk < p.SS; sk += W) out[sk] = (uint32_t)X[p.T[p.oCs + sk]];
         L.cursor = 1;
     }
     const uint32_t* last = out + (size_t)(L.cursor - 1) * p.SS;
     for (int i = (int)L.cursor; i < p.K; ++i)
-        for (int sk = l; sk < p.SS; sk += G) out[(size_t)i * p.SS + sk] = last[sk];
+        for (int sk = l; sk < p.SS; sk += W) out[(size_t)i * p.SS + sk] = last[sk];
     L.t = p.tmax + (double)0.1f;
     L.cursor = (uint32_t)p.K;
     L.absorbed = 1;
 }
 
 // One adaptive leap attempt (PreCalculations, T.cu:1568-2093).
-template <int G, int PFM = 3>
+template <int G, int W, int PFM = 3>
 __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V, int l,
                                      const float* __restrict__ recip) {
     if (L.t >= p.tmax) return LEAP_DONE;
+    const int la = l & (G - 1);              // the algorithm's lane this one stands for
+    const bool own = l < G;                  // one lane per algorithm lane counts
     int32_t* X = V.Xb + (L.xb ? p.S : 0);
     int32_t* X1 = V.Xb + (L.xb ? 0 : p.S);
     float P, PC;
     if (pmode<PFM>(kuse(p.pfast)) == 1) {
-        gfactors<G>(p, X, V.F, l);
+        gfactors<W>(p, X, V.F, l);
         gsync();
     }
-    gprops<G, PFM>(p, X, V.F, L.crate, V.A, l, P, PC);
+    gprops<G, W, PFM>(p, X, V.F, L.crate, V.A, l, P, PC);
     gsync();
-    P = gscan<G>(P, l);
-    PC = gscan<G>(PC, l);
-    const float a0 = gbcast_last<G>(P, l);
-    const float a0c = gbcast_last<G>(PC, l);
+    P = gscan<G>(P, la);
+    PC = gscan<G>(PC, la);
+    const float a0 = gbcast_last<G>(P, la);
+    const float a0c = gbcast_last<G>(PC, la);
     CTL_PHASE(PH_PROPS);
-    if (a0 == 0.0f) { gabsorb<G>(p, L, X, l); return LEAP_ABSORB; }
+    if (a0 == 0.0f) { gabsorb<W>(p, L, X, l); return LEAP_ABSORB; }
     // tau' (T.cu:1860-1922): the one-lane kernel's per-species values, min over lanes
     float tau1 = 3.40282347e+38f;
     const ctab_u32 TC = CT_U32(p.T);
-    const int nrs = (p.S + G - 1) / G;
+    const int nrs = (p.S + W - 1) / W;
     const uint32_t* E = p.T + p.oVRe + l;
     const uint32_t* SPI = p.T + p.oSPI + l;
     for (int r = 0; r < nrs; ++r) {
         const uint32_t len = TC[p.oVRm + r];
-        const uint32_t spw = SPI[r * G];             // species | HOR << 16 | HORtype << 24
+        const uint32_t spw = SPI[r * W];             // species | HOR << 16 | HORtype << 24
         float mu = 0.0f, sg = 0.0f;
         if (kuse(p.vhalf)) {
             // entries (coefficient as FP16 << 16 | byte offset of A[reaction]):
@@ -667,7 +757,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
                 uint32_t e[4];
                 int32_t u[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) e[i] = E[(k + i) * G];
+                for (int i = 0; i < 4; ++i) e[i] = E[(k + i) * W];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) u[i] = *reinterpret_cast<const int32_t*>(Ab + (e[i] & 0xffffu));
 #pragma unroll
@@ -685,7 +775,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
             for (uint32_t k = 0; k < len; k += 4) {  // len is a multiple of 4
                 uint32_t e[4], u[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) e[i] = E[(k + i) * G];
+                for (int i = 0; i < 4; ++i) e[i] = E[(k + i) * W];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) u[i] = V.A[e[i] & 0xffffu];
 #pragma unroll
@@ -698,7 +788,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
                 }
             }
         }
-        E += len * G;
+        E += len * W;
         if (mu == 0.0f || sg == 0.0f) continue;      // no var entries (no species included)
         const int32_t x = X[spw & 0xffffu];
         const float ex = p.eps * (float)x;
@@ -712,25 +802,25 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         const float tmp = t3 < t4 ? t3 : t4;
         if (tmp < tau1) tau1 = tmp;
     }
-    tau1 = gmin<G>(tau1);
+    tau1 = gmin<W>(tau1);
     CTL_PHASE(PH_TAU1);
     if (tau1 < p.ssa_factor / a0) { L.switches++; return LEAP_SWITCH; }      // T.cu:1935-1941
     uint32_t e = L.evc++;
     grng_event(L.gg, e);
     float tau2 = 3.40282347e+38f;
-    if (a0c > 0.0f) tau2 = u32_exp(grng_u32<G>(L.gg, l)) / a0c;                                // T.cu:1962-1965
+    if (a0c > 0.0f) tau2 = u32_exp(grng_u32<W>(L.gg, l)) / a0c;                                // T.cu:1962-1965
     float tau = tau1 < tau2 ? tau1 : tau2;
     int pick = -1;
     if (tau1 > tau2) {                                                         // T.cu:1993-2006
-        const float w = u32_oc(grng_u32<G>(L.gg, l)) * a0c;
+        const float w = u32_oc(grng_u32<W>(L.gg, l)) * a0c;
         float Q = 0.0f;
-        for (int j = l; j < p.R; j += G) {
+        for (int j = la; j < p.R; j += G) {
             const uint32_t u = V.A[j];
             if ((u & 0x80000000u) || j == 0) Q = Q + aval(u);
         }
         const float Qown = Q;
-        Q = gscan<G>(Q, l);
-        pick = gselect<G>(p, V.A, Qown, Q, w, l, 2);
+        Q = gscan<G>(Q, la);
+        pick = gselect<G>(p, V.A, Qown, Q, w, la, 2);
     }
     CTL_PHASE(PH_PICK);
     uint64_t fired = 0;
@@ -746,7 +836,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         if (l == 0) *V.qn = 0u;
         gsync();
         double cum = 0.0, pos = (double)exp_rv(L.lg);
-        L.gaps++;
+        if (own) L.gaps++;
         // The lane's second event position is drawn now, with the first, by
         // every lane at once; drawn inside the loop below it would cost the
         // wavefront a divergent draw for almost every reaction round.  It is
@@ -756,7 +846,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         bool have2 = true;
         const int nit = (p.R + G - 1) / G;
         for (int i = 0; i < nit; ++i) {
-            const int j = l + i * G;
+            const int j = la + i * G;
             bool need = false;
             {                                          // past R: the zero padding of A and Kc
                 const uint32_t u = V.A[j];
@@ -776,19 +866,21 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
                     } else {
                         pos = pos + (double)exp_rv(L.lg);
                     }
-                    L.gaps++;
+                    if (own) L.gaps++;
                 }
-                V.Kc[j] = k;                         // a queued reaction's count is drawn below
-                fk += (uint32_t)k;
+                if (own) {
+                    V.Kc[j] = k;                     // a queued reaction's count is drawn below
+                    fk += (uint32_t)k;
+                }
             }
             // the queue's order is free: each count comes from its reaction's own stream
-            if (need) Q[atomicAdd(V.qn, 1u)] = (uint16_t)j;
+            if (need && own) Q[atomicAdd(V.qn, 1u)] = (uint16_t)j;
         }
         gsync();
         CTL_PHASE(PH_COUNTS);
         const uint32_t nq = *V.qn;
         uint64_t f = fk;
-        for (uint32_t qi = (uint32_t)l; qi < nq; qi += G) {
+        for (uint32_t qi = (uint32_t)l; qi < nq; qi += W) {
             const int j = Q[qi];
             const float lam = tau * __uint_as_float(V.A[j]);
             Rng gr{};
@@ -808,7 +900,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         const uint32_t* F = p.T + p.oFRe + l;
         for (int r = 0; r < nrs; ++r) {
             const uint32_t len = TC[p.oFRm + r];
-            const uint32_t sp = SPI[r * G] & 0xffffu;
+            const uint32_t sp = SPI[r * W] & 0xffffu;
             if (sp < (uint32_t)p.S) {
                 int64_t x = X[sp];
                 bool bs = false;
@@ -816,7 +908,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
                     uint32_t e[4];
                     int32_t kc[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) e[i] = F[(k + i) * G];
+                    for (int i = 0; i < 4; ++i) e[i] = F[(k + i) * W];
 #pragma unroll
                     for (int i = 0; i < 4; ++i) kc[i] = V.Kc[e[i] & 0xffffu];
 #pragma unroll
@@ -828,10 +920,10 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
                 X1[sp] = (int32_t)x;
                 bad = bad || bs;
             }
-            F += len * G;
+            F += len * W;
         }
-        fired = gsum64<G>(f);
-        const bool any_bad = gballot<G>(bad) != 0;
+        fired = gsum64<W>(f);
+        const bool any_bad = gballot<W>(bad) != 0;
         gsync();
         CTL_PHASE(PH_UPDATE);
         if (!any_bad) break;
@@ -845,7 +937,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
             uint32_t* out = p.storage + (size_t)L.sim * p.K * p.SS;
             while (i < (uint32_t)p.K && tn >= p.ts[i]) {
                 const double ti = p.ts[i];
-                for (int sk = l; sk < p.SS; sk += G) {
+                for (int sk = l; sk < p.SS; sk += W) {
                     const int sp = (int)p.T[p.oCs + sk];
                     const int32_t d = X1[sp] - X[sp];
                     uint32_t val = (uint32_t)X[sp];
@@ -863,7 +955,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
     L.xb ^= 1u;
     if (kuse(p.nfs) > 0) {               // feeds (T.cu:2072-2079)
         int32_t* Xn = V.Xb + (L.xb ? p.S : 0);
-        for (int u = l; u < p.nfs; u += G) Xn[p.fs[u]] = (int32_t)L.fvrow[u];
+        for (int u = l; u < p.nfs; u += W) Xn[p.fs[u]] = (int32_t)L.fvrow[u];
         gsync();
     }
     L.t = L.t + (double)tau;
@@ -880,19 +972,20 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
 // group's LDS), so the steps and their draws are those of one call.  After
 // the fired reaction only its dependent propensities are recomputed (same
 // values as recomputing all).  Returns true on absorption.
-template <int G, int PFM = 3>
+template <int G, int W, int PFM = 3>
 __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView& V, int l, int nmax) {
     int32_t* X = V.Xb + (L.xb ? p.S : 0);
+    const int la = l & (G - 1);              // the algorithm's lane this one stands for
     if (L.ssa_left == 0) {
         grng_event(L.gg, L.evc++);
         L.tacc = 0.0;
         L.ssa_left = p.ssa_steps;
         if (pmode<PFM>(kuse(p.pfast)) == 1) {
-            gfactors<G>(p, X, V.F, l);
+            gfactors<W>(p, X, V.F, l);
             gsync();
         }
         float P, PC;
-        gprops<G, PFM>(p, X, V.F, L.crate, V.A, l, P, PC);
+        gprops<G, W, PFM>(p, X, V.F, L.crate, V.A, l, P, PC);
         gsync();
     }
     CTL_PHASE(PH_SSA_OPEN);
@@ -904,18 +997,18 @@ __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView
         for (int r0 = 0; r0 < nrp; r0 += 4) {          // padding adds an exact 0
             uint32_t u[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) u[i] = r0 + i < nrp ? V.A[l + (r0 + i) * G] : 0u;
+            for (int i = 0; i < 4; ++i) u[i] = r0 + i < nrp ? V.A[la + (r0 + i) * G] : 0u;
 #pragma unroll
             for (int i = 0; i < 4; ++i) P = P + aval(u[i]);
         }
         const float Pown = P;
-        P = gscan<G>(P, l);
-        const float a0 = gbcast_last<G>(P, l);
-        if (a0 == 0.0f) { gabsorb<G>(p, L, X, l); L.ssa_left = 0; return true; }
-        const float r1 = u32_oc(grng_u32<G>(L.gg, l)) * a0;
-        const int j = gselect<G>(p, V.A, Pown, P, r1, l, 0);
-        if (j < 0) { gabsorb<G>(p, L, X, l); L.ssa_left = 0; return true; }    // unreachable for finite a0
-        const float dt = u32_exp(grng_u32<G>(L.gg, l)) / a0;
+        P = gscan<G>(P, la);
+        const float a0 = gbcast_last<G>(P, la);
+        if (a0 == 0.0f) { gabsorb<W>(p, L, X, l); L.ssa_left = 0; return true; }
+        const float r1 = u32_oc(grng_u32<W>(L.gg, l)) * a0;
+        const int j = gselect<G>(p, V.A, Pown, P, r1, la, 0);
+        if (j < 0) { gabsorb<W>(p, L, X, l); L.ssa_left = 0; return true; }    // unreachable for finite a0
+        const float dt = u32_exp(grng_u32<W>(L.gg, l)) / a0;
         CTL_PHASE(PH_SSA_SELECT);
         tacc = tacc + (double)dt;
         const double tn = L.t + tacc;
@@ -923,7 +1016,7 @@ __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView
         if (i < (uint32_t)p.K && tn > p.ts[i]) {                               // T.cu:2213-2236
             uint32_t* out = p.storage + (size_t)L.sim * p.K * p.SS;
             while (i < (uint32_t)p.K && tn > p.ts[i]) {
-                for (int sk = l; sk < p.SS; sk += G) out[(size_t)i * p.SS + sk] = (uint32_t)X[p.T[p.oCs + sk]];
+                for (int sk = l; sk < p.SS; sk += W) out[(size_t)i * p.SS + sk] = (uint32_t)X[p.T[p.oCs + sk]];
                 ++i;
             }
             L.cursor = i;
@@ -932,7 +1025,7 @@ __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView
         const uint32_t f1 = p.T[p.oFp + j + 1];
         const int pm = pmode<PFM>(kuse(p.pfast));
         const bool fac = pm == 1;
-        for (uint32_t h = p.T[p.oFp + j] + (uint32_t)l; h < f1; h += G) {
+        for (uint32_t h = p.T[p.oFp + j] + (uint32_t)l; h < f1; h += W) {
             const uint32_t ent = p.T[p.oFe + h];
             const int s = (int)(ent & 0xffffu);
             const int v = (int)(int16_t)(ent >> 16);
@@ -948,7 +1041,7 @@ __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView
         if (fac) {
             // dependent records {r, factor index 0, factor index 1, 0}: one 16-byte load each
             const uint4* DR = reinterpret_cast<const uint4*>(p.T + p.oDR);
-            for (uint32_t d = d0 + (uint32_t)l; d < d1; d += G) {
+            for (uint32_t d = d0 + (uint32_t)l; d < d1; d += W) {
                 const uint4 rec = DR[d];
                 const int r = (int)rec.x;
                 const uint32_t u0 = V.F[rec.y], u1 = V.F[rec.z];
@@ -961,7 +1054,7 @@ __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView
             // dependent records {r, reactant entry 0, entry 1, 0} read from the state
             const uint4* DR = reinterpret_cast<const uint4*>(p.T + p.oDR);
             const uint32_t nc = (uint32_t)p.nc;
-            for (uint32_t d = d0 + (uint32_t)l; d < d1; d += G) {
+            for (uint32_t d = d0 + (uint32_t)l; d < d1; d += W) {
                 const uint4 rec = DR[d];
                 const int r = (int)rec.x;
                 float a = L.crate[r];
@@ -970,7 +1063,7 @@ __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView
                 V.A[r] = __float_as_uint(a) | (c ? 0x80000000u : 0u);
             }
         } else {
-            for (uint32_t d = d0 + (uint32_t)l; d < d1; d += G) {
+            for (uint32_t d = d0 + (uint32_t)l; d < d1; d += W) {
                 const int r = (int)p.T[p.oDe + d];
                 bool crit;
                 const float a = gprop(p, X, L.crate, r, crit);
@@ -990,10 +1083,10 @@ __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView
 }
 
 // One whole SSA burst.
-template <int G, int PFM = 3>
+template <int G, int W, int PFM = 3>
 __device__ __forceinline__ bool gssa(const KParams& p, GLane& L, const GView& V, int l) {
     L.ssa_left = 0;
-    return gssa_run<G, PFM>(p, L, V, l, p.ssa_steps);
+    return gssa_run<G, W, PFM>(p, L, V, l, p.ssa_steps);
 }
 
 __device__ __forceinline__ const float* grates(const KParams& p, int sim) {
@@ -1001,11 +1094,11 @@ __device__ __forceinline__ const float* grates(const KParams& p, int sim) {
 }
 
 // Next simulation from the queue (PrepareVariables, T.cu:1269-1297).
-template <int G>
+template <int W>
 __device__ __forceinline__ bool gfetch(const KParams& p, GLane& L, const GView& V, int l) {
     uint32_t q = 0;
     if (l == 0) q = atomicAdd(p.next_sim, 1u);
-    q = __shfl(q, 0, G);
+    q = __shfl(q, 0, W);
     if (q >= (uint32_t)p.n) { L.sim = -2; return false; }
     L.sim = (int)q;
     L.t = 0.0;
@@ -1021,7 +1114,7 @@ __device__ __forceinline__ bool gfetch(const KParams& p, GLane& L, const GView& 
     L.gg.sim = L.lg.sim = p.sim_base + q;
     L.gg.cb = GRNG_NONE;
     L.lg.pos = 4;
-    for (int s = l; s < p.S; s += G)
+    for (int s = l; s < p.S; s += W)
         V.Xb[s] = (int32_t)(p.x0_bcast ? p.x0_bcast[s] : p.x0_sims[(size_t)(q / (uint32_t)p.x0_div) * p.S + s]);
     L.crate = grates(p, (int)q);
     L.fvrow = p.nfs > 0 ? p.fv + (size_t)(q / (uint32_t)p.fv_div) * p.nfs : nullptr;
@@ -1029,12 +1122,12 @@ __device__ __forceinline__ bool gfetch(const KParams& p, GLane& L, const GView& 
     return true;
 }
 
-template <int G>
+template <int W>
 __device__ __forceinline__ void gfinish(const KParams& p, GLane& L, const GView& V, int l) {
     const int32_t* X = V.Xb + (L.xb ? p.S : 0);
-    const uint64_t pois = gsum64<G>(L.poisson);
-    const uint64_t gaps = gsum64<G>(L.gaps);
-    for (int s = l; s < p.S; s += G) p.xfinal[(size_t)L.sim * p.S + s] = X[s];
+    const uint64_t pois = gsum64<W>(L.poisson);
+    const uint64_t gaps = gsum64<W>(L.gaps);
+    for (int s = l; s < p.S; s += W) p.xfinal[(size_t)L.sim * p.S + s] = X[s];
     if (l == 0) {
         ctl_sim_stat st;
         st.firings = L.firings;
@@ -1073,10 +1166,10 @@ constexpr int GBURST_WAIT = 24;
 // ---------------------------------------------------------------------------
 
 // Writes the group's registers to the slot arrays of its region's slot s0.
-template <int G>
+template <int W>
 __device__ __forceinline__ void gstage_put(const KParams& p, const GLane& L, int s0, int l) {
-    p.st->poisson[(size_t)s0 * G + l] = L.poisson;
-    p.st->gaps[(size_t)s0 * G + l] = L.gaps;
+    p.st->poisson[(size_t)s0 * W + l] = L.poisson;
+    p.st->gaps[(size_t)s0 * W + l] = L.gaps;
     if (l == 0) {
         p.st->sim[s0] = L.sim;
         p.st->t[s0] = L.t;
@@ -1098,11 +1191,11 @@ __device__ __forceinline__ void gstage_put(const KParams& p, const GLane& L, int
 
 // Takes over the simulation of slot s0: its registers, rate and feed rows and
 // the position in its group stream.
-template <int G>
+template <int W>
 __device__ __forceinline__ void gstage_get(const KParams& p, GLane& L, int s0, int l) {
     L.sim = p.st->sim[s0];
-    L.poisson = p.st->poisson[(size_t)s0 * G + l];
-    L.gaps = p.st->gaps[(size_t)s0 * G + l];
+    L.poisson = p.st->poisson[(size_t)s0 * W + l];
+    L.gaps = p.st->gaps[(size_t)s0 * W + l];
     L.absorbed = 0;
     if (L.sim < 0) return;
     L.t = p.st->t[s0];
@@ -1131,7 +1224,7 @@ __device__ __forceinline__ void gstage_get(const KParams& p, GLane& L, int s0, i
 // no region of the workgroup holds a simulation; else the new region of
 // this lane's group in *next and whether any region moves to other lanes in
 // *moves (the same for the whole workgroup).
-template <int G>
+template <int W>
 __device__ __forceinline__ bool gregroup(int key, int reg, uint32_t* cnt, uint32_t* perm, int l, int* next,
                                          bool* moves) {
     const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6), nw = (int)(blockDim.x >> 6);
@@ -1152,49 +1245,54 @@ __device__ __forceinline__ bool gregroup(int key, int reg, uint32_t* cnt, uint32
     for (int w = 0; w < wave; ++w) pos += cnt[w * 3 + key];
     if (l == 0) perm[pos + rank] = (uint32_t)reg;
     __syncthreads();
-    const int nreg = (int)(blockDim.x / G);
+    const int nreg = (int)(blockDim.x / W);
     bool mv = false;
     for (int q = 0; q < nreg; ++q) mv = mv || perm[q] != (uint32_t)q;
     *moves = mv;
-    *next = (int)perm[threadIdx.x / G];
+    *next = (int)perm[threadIdx.x / W];
     return true;
 }
 
-// Persistent group kernel: p.ns lanes = p.ns / G group slots, each pulling
+// Waves per SIMD the group kernels are compiled for.  W = G: G = 8, 16 and 32
+// for four (128 VGPRs, a few bytes of scratch), measured +9 % at G = 16 and
+// +4 % at G = 32 on the 100x200 network, +24 % at G = 8 on the 50x100 sweep
+// network; G = 4 groups are bounded by LDS instead, and G = 64 would spill
+// heavily.  W > G serves runs that leave the chip short of wavefronts.
+__host__ __device__ constexpr int gwaves(int G, int W) {
+    return W > G ? (W == 64 ? 2 : 4) : (G == 8 || G == 16 || G == 32 ? 4 : 1);
+}
+
+// Persistent group kernel: p.ns lanes = p.ns / W group slots, each pulling
 // simulations from the queue; a launch runs up to p.iters iterations per
 // group (a leap attempt, or SSA steps), then parks the group's state in the
-// slot arrays for the next launch.  Without regrouping (RG false: G = 64, or
+// slot arrays for the next launch.  Without regrouping (RG false: W = 64, or
 // p.compact = 0) a group that switched to SSA holds its whole burst until a second
 // group of the wavefront switches too (or it has waited GBURST_WAIT
 // iterations, or every group still running is waiting), so that bursts run
 // side by side.  Either way each simulation's events and draws are its own;
 // only the order in which the lanes serve the simulations moves.
-// G = 8, 16 and 32 are compiled for four waves per SIMD (128 VGPRs, a few
-// bytes of scratch): measured +9 % at G = 16 and +4 % at G = 32 on the
-// 100x200 network, +24 % at G = 8 on the 50x100 sweep network.  G = 4
-// groups are bounded by LDS instead, and G = 64 would spill heavily.
-template <int G, bool RG, int PF>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G == 8 || G == 16 || G == 32 ? 4 : 1))) void group_kernel(KParams p) {
+template <int G, int W, bool RG, int PF>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gwaves(G, W)))) void group_kernel(KParams p) {
     extern __shared__ uint32_t smem[];
     __shared__ float recip[64];
     __shared__ uint32_t rg_cnt[12];
-    __shared__ uint32_t rg_perm[256 / G];
+    __shared__ uint32_t rg_perm[256 / W];
     for (int i = threadIdx.x; i < 64; i += blockDim.x) recip[i] = c_recip[i];
     __syncthreads();
-    const int l = (int)(threadIdx.x & (unsigned)(G - 1));
-    const int nreg = (int)(blockDim.x / G);
-    int gib = (int)(threadIdx.x / G);
+    const int l = (int)(threadIdx.x & (unsigned)(W - 1));
+    const int nreg = (int)(blockDim.x / W);
+    int gib = (int)(threadIdx.x / W);
     const size_t gw = group_lds_words(p.S, p.R, G);
-    constexpr bool rg = RG && G < 64;     // the host launches RG only with p.compact > 0 and several wavefronts
+    constexpr bool rg = RG && W < 64;     // the host launches RG only with p.compact > 0 and several wavefronts
     GLane L;
     L.slot = (int)blockIdx.x * nreg + gib;
     CTL_PHASE_START();
-    if (L.slot * G >= p.ns) return;                  // whole workgroups when regrouping
+    if (L.slot * W >= p.ns) return;                  // whole workgroups when regrouping
     GView V = group_view(smem + (size_t)gib * gw, p.S, p.R, G);
-    gzero_pad<G>(V, p.R, l);
+    gzero_pad<G, W>(V, p.R, l);
     L.gg.k0 = L.lg.k0 = p.key0;
     L.gg.k1 = L.lg.k1 = p.key1;
-    L.lg.tag = 1u + (uint32_t)l;
+    L.lg.tag = 1u + (uint32_t)(l & (G - 1));
     L.tacc = 0.0;
     L.ssa_left = 0;
     L.ssa_mode = 0;
@@ -1217,12 +1315,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G == 8 || G
         L.switches = p.st->switches[s0];
         L.absorbed = 0;
         L.ssa_mode = kuse(p.force_ssa);
-        L.poisson = p.st->poisson[(size_t)s0 * G + l];
-        L.gaps = p.st->gaps[(size_t)s0 * G + l];
+        L.poisson = p.st->poisson[(size_t)s0 * W + l];
+        L.gaps = p.st->gaps[(size_t)s0 * W + l];
         L.gg.sim = L.lg.sim = p.sim_base + (uint32_t)L.sim;
         L.gg.cb = GRNG_NONE;
         L.lg.pos = 4;
-        for (int s = l; s < p.S; s += G) V.Xb[s] = p.X[(size_t)s0 * p.S + s];
+        for (int s = l; s < p.S; s += W) V.Xb[s] = p.X[(size_t)s0 * p.S + s];
         L.crate = grates(p, L.sim);
         L.fvrow = p.nfs > 0 ? p.fv + (size_t)(L.sim / p.fv_div) * p.nfs : nullptr;
         gsync();
@@ -1237,54 +1335,54 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G == 8 || G
                 const int key = L.sim == -2 ? 2 : (L.sim >= 0 ? L.ssa_mode : kuse(p.force_ssa));
                 int ng;
                 bool moves;
-                if (!gregroup<G>(key, gib, rg_cnt, rg_perm, l, &ng, &moves)) break;
+                if (!gregroup<W>(key, gib, rg_cnt, rg_perm, l, &ng, &moves)) break;
                 // a group whose region stays on its lanes keeps its registers;
                 // the others hand their state over through the slot arrays
                 if (moves) {
                     const bool move = ng != gib;
-                    if (move) gstage_put<G>(p, L, L.slot, l);
+                    if (move) gstage_put<W>(p, L, L.slot, l);
                     __syncthreads();
                     if (move) {
                         gib = ng;
                         L.slot = (int)blockIdx.x * nreg + gib;
-                        gstage_get<G>(p, L, L.slot, l);
+                        gstage_get<W>(p, L, L.slot, l);
                         V = group_view(smem + (size_t)gib * gw, p.S, p.R, G);
                     }
                 }
                 CTL_PHASE(PH_REGROUP);
             }
             if (L.sim == -2) continue;
-            if (L.sim < 0 && !gfetch<G>(p, L, V, l)) continue;
+            if (L.sim < 0 && !gfetch<W>(p, L, V, l)) continue;
             if (L.ssa_mode) {
                 CTL_PHASE(PH_PRE_SSA);
                 if (kuse(p.force_ssa) && L.ssa_left == 0 && L.t >= p.tmax) {
-                    gfinish<G>(p, L, V, l);
-                } else if (gssa_run<G, PF>(p, L, V, l, p.ssa_chunk)) {
-                    gfinish<G>(p, L, V, l);
+                    gfinish<W>(p, L, V, l);
+                } else if (gssa_run<G, W, PF>(p, L, V, l, p.ssa_chunk)) {
+                    gfinish<W>(p, L, V, l);
                 } else if (L.ssa_left == 0 && !kuse(p.force_ssa)) {
                     L.ssa_mode = 0;
                 }
             } else {
                 CTL_PHASE(PH_PRE_LEAP);
-                const int r = gleap<G, PF>(p, L, V, l, recip);
+                const int r = gleap<G, W, PF>(p, L, V, l, recip);
                 if (r == LEAP_DONE || r == LEAP_ABSORB) {
-                    gfinish<G>(p, L, V, l);
+                    gfinish<W>(p, L, V, l);
                 } else if (r == LEAP_SWITCH) {
                     L.ssa_mode = 1;
                 }
             }
             continue;
         }
-        if (L.sim < 0 && !gfetch<G>(p, L, V, l)) break;
+        if (L.sim < 0 && !gfetch<W>(p, L, V, l)) break;
         if (kuse(p.force_ssa)) {
-            if (L.t >= p.tmax || gssa<G, PF>(p, L, V, l)) gfinish<G>(p, L, V, l);
+            if (L.t >= p.tmax || gssa<G, W, PF>(p, L, V, l)) gfinish<W>(p, L, V, l);
             continue;
         }
         if (!pend) {
             CTL_PHASE(PH_PRE_LEAP);
-            const int r = gleap<G, PF>(p, L, V, l, recip);
+            const int r = gleap<G, W, PF>(p, L, V, l, recip);
             if (r == LEAP_DONE || r == LEAP_ABSORB) {
-                gfinish<G>(p, L, V, l);
+                gfinish<W>(p, L, V, l);
             } else if (r == LEAP_SWITCH) {
                 pend = true;
                 waited = 0;
@@ -1293,7 +1391,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G == 8 || G
             ++waited;
         }
         bool go = pend;
-        if (G < 64) {
+        if (W < 64) {
             const uint64_t lead = __ballot(l == 0);            // groups still in the loop
             const uint64_t pm = __ballot(pend && l == 0);       // ... waiting for a burst
             go = pm != 0 && (__popcll(pm) >= 2 || pm == lead || __ballot(pend && waited >= GBURST_WAIT) != 0);
@@ -1301,7 +1399,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G == 8 || G
         if (go && pend) {
             pend = false;
             CTL_PHASE(PH_PRE_SSA);
-            if (gssa<G, PF>(p, L, V, l)) gfinish<G>(p, L, V, l);
+            if (gssa<G, W, PF>(p, L, V, l)) gfinish<W>(p, L, V, l);
         }
     }
     // before parking: the burst of a switched simulation runs to its end (a
@@ -1309,17 +1407,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G == 8 || G
     // force-SSA mode)
     if (rg) {
         if (L.sim >= 0 && (L.ssa_left > 0 || (L.ssa_mode && !kuse(p.force_ssa))) &&
-            gssa_run<G, PF>(p, L, V, l, L.ssa_left > 0 ? L.ssa_left : p.ssa_steps))
-            gfinish<G>(p, L, V, l);
-    } else if (pend && gssa<G, PF>(p, L, V, l)) {
-        gfinish<G>(p, L, V, l);
+            gssa_run<G, W, PF>(p, L, V, l, L.ssa_left > 0 ? L.ssa_left : p.ssa_steps))
+            gfinish<W>(p, L, V, l);
+    } else if (pend && gssa<G, W, PF>(p, L, V, l)) {
+        gfinish<W>(p, L, V, l);
     }
     const int s0 = L.slot;
     if (L.sim >= 0) {                    // park: state to the slot arrays
         const int32_t* X = V.Xb + (L.xb ? p.S : 0);
-        for (int s = l; s < p.S; s += G) p.X[(size_t)s0 * p.S + s] = X[s];
-        p.st->poisson[(size_t)s0 * G + l] = L.poisson;
-        p.st->gaps[(size_t)s0 * G + l] = L.gaps;
+        for (int s = l; s < p.S; s += W) p.X[(size_t)s0 * p.S + s] = X[s];
+        p.st->poisson[(size_t)s0 * W + l] = L.poisson;
+        p.st->gaps[(size_t)s0 * W + l] = L.gaps;
         if (l == 0) {
             p.st->t[s0] = L.t;
             p.st->cursor[s0] = L.cursor;
@@ -1338,26 +1436,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G == 8 || G
 
 // Host: appends the lane-interleaved round streams (KParams::oPRm ..) of a
 // group kernel with G lanes to the packed table buffer T.
-inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, const Model& m,
+inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, int W, const Model& m,
                                  const std::vector<uint32_t>& FSptr, const std::vector<uint32_t>& FSent,
                                  const std::vector<uint32_t>& Dent) {
-    // Item order[r * G + l] (-1: none) goes to lane l of round r.  fixed > 0:
+    // Item order[r * B + l] (-1: none) goes to lane l of round r of B lanes.  fixed > 0:
     // every round has exactly that many entries per lane; else the round's
     // longest list rounded up to a multiple of quantum.
-    auto rounds = [&](const std::vector<int>& order, const std::vector<uint32_t>& ptr,
+    auto rounds = [&](int B, const std::vector<int>& order, const std::vector<uint32_t>& ptr,
                       const std::vector<uint32_t>& ent, int& om, int& oe, uint32_t quantum, uint32_t fixed,
                       uint32_t pad) {
-        const int nr = (int)(order.size() / (size_t)G);
+        const int nr = (int)(order.size() / (size_t)B);
         auto cnt = [&](int i) { return i < 0 ? 0u : ptr[i + 1] - ptr[i]; };
         std::vector<uint32_t> len((size_t)nr, 0u), e;
         for (int r = 0; r < nr; ++r) {
             uint32_t mx = 0;
-            for (int l = 0; l < G; ++l) mx = std::max(mx, cnt(order[(size_t)r * G + l]));
+            for (int l = 0; l < B; ++l) mx = std::max(mx, cnt(order[(size_t)r * B + l]));
             mx = fixed ? fixed : (mx + quantum - 1) / quantum * quantum;
             len[r] = mx;
             for (uint32_t k = 0; k < mx; ++k)
-                for (int l = 0; l < G; ++l) {
-                    const int i = order[(size_t)r * G + l];
+                for (int l = 0; l < B; ++l) {
+                    const int i = order[(size_t)r * B + l];
                     e.push_back(k < cnt(i) ? ent[ptr[i] + k] : pad);
                 }
         }
@@ -1390,9 +1488,9 @@ inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, co
     if (p.pfast == 1) {
         std::vector<uint32_t> fent(m.Lent.size());
         for (size_t h = 0; h < m.Lent.size(); ++h) fent[h] = findex(m.Lent[h]);
-        rounds(rorder, m.Lptr, fent, p.oPRm, p.oPRe, 1, 2, one);
+        rounds(G, rorder, m.Lptr, fent, p.oPRm, p.oPRe, 1, 2, one);
     } else {
-        rounds(rorder, m.Lptr, m.Lent, p.oPRm, p.oPRe, 1, p.pfast == 2 ? 2 : 0, 0u);
+        rounds(G, rorder, m.Lptr, m.Lent, p.oPRm, p.oPRe, 1, p.pfast == 2 ? 2 : 0, 0u);
     }
     p.oDR = 0;
     if (p.pfast) {                        // dependent records, 16-byte aligned
@@ -1410,7 +1508,7 @@ inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, co
     // species by entry count, longest first, so that a round's lanes carry
     // lists of similar length (tau' is a minimum and the update is per
     // species, so the species-to-lane map is free)
-    std::vector<int> sorder((size_t)((m.S + G - 1) / G) * G, -1);
+    std::vector<int> sorder((size_t)((m.S + W - 1) / W) * W, -1);
     for (int i = 0; i < m.S; ++i) sorder[i] = i;
     std::stable_sort(sorder.begin(), sorder.begin() + m.S, [&](int a, int b) {
         return std::max(m.Vptr[a + 1] - m.Vptr[a], FSptr[a + 1] - FSptr[a]) >
@@ -1437,11 +1535,11 @@ inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, co
             const _Float16 hv = (_Float16)(float)(int16_t)(m.Vent[h] >> 16);
             vent[h] = (uint32_t)__builtin_bit_cast(uint16_t, hv) << 16 | (m.Vent[h] & 0xffffu) * 4u;
         }
-        rounds(sorder, m.Vptr, vent, p.oVRm, p.oVRe, 4, 0, (uint32_t)m.R * 4u);   // padding: A[R] = 0
+        rounds(W, sorder, m.Vptr, vent, p.oVRm, p.oVRe, 4, 0, (uint32_t)m.R * 4u);   // padding: A[R] = 0
     } else {
-        rounds(sorder, m.Vptr, m.Vent, p.oVRm, p.oVRe, 4, 0, (uint32_t)m.R);       // padding: the zero slot A[R]
+        rounds(W, sorder, m.Vptr, m.Vent, p.oVRm, p.oVRe, 4, 0, (uint32_t)m.R);       // padding: the zero slot A[R]
     }
-    rounds(sorder, FSptr, FSent, p.oFRm, p.oFRe, 4, 0, 0u);
+    rounds(W, sorder, FSptr, FSent, p.oFRm, p.oFRe, 4, 0, 0u);
 }
 
 }  // namespace ctl

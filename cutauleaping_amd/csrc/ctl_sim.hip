@@ -140,33 +140,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
     store_lane(p, L);
 }
 
-// The group kernel instance for G lanes per simulation, with or without
-// regrouping, for propensity mode pf (KParams::pfast: 0, 1 or 2).
-template <int G, bool RG>
+// The group kernel instance for the G-lane algorithm on W lanes per
+// simulation, with or without regrouping, for propensity mode pf
+// (KParams::pfast: 0, 1 or 2).  Regrouping instances exist for W = G < 64.
+template <int G, int W, bool RG>
 const void* group_kernel_fn_p(int pf) {
     switch (pf) {
-        case 1: return (const void*)group_kernel<G, RG, 1>;
-        case 2: return (const void*)group_kernel<G, RG, 2>;
+        case 1: return (const void*)group_kernel<G, W, RG, 1>;
+        case 2: return (const void*)group_kernel<G, W, RG, 2>;
     }
-    return (const void*)group_kernel<G, RG, 0>;
+    return (const void*)group_kernel<G, W, RG, 0>;
 }
 
 template <int G>
-const void* group_kernel_fn_g(bool rg, int pf) {
-    if constexpr (G < 64) {
-        if (rg) return group_kernel_fn_p<G, true>(pf);
+const void* group_kernel_fn_g(int W, bool rg, int pf) {
+    if (W == G) {
+        if constexpr (G < 64) {
+            if (rg) return group_kernel_fn_p<G, G, true>(pf);
+        }
+        return group_kernel_fn_p<G, G, false>(pf);
     }
-    return group_kernel_fn_p<G, false>(pf);
+    if constexpr (G < 16) {
+        if (W == 16) return group_kernel_fn_p<G, 16, false>(pf);
+    }
+    if constexpr (G < 32) {
+        if (W == 32) return group_kernel_fn_p<G, 32, false>(pf);
+    }
+    if constexpr (G < 64) {
+        if (W == 64) return group_kernel_fn_p<G, 64, false>(pf);
+    }
+    return nullptr;
 }
 
-const void* group_kernel_fn(int G, bool rg, int pf) {
+const void* group_kernel_fn(int G, int W, bool rg, int pf) {
     switch (G) {
-        case 2: return group_kernel_fn_g<2>(rg, pf);
-        case 4: return group_kernel_fn_g<4>(rg, pf);
-        case 8: return group_kernel_fn_g<8>(rg, pf);
-        case 16: return group_kernel_fn_g<16>(rg, pf);
-        case 32: return group_kernel_fn_g<32>(rg, pf);
-        case 64: return group_kernel_fn_g<64>(false, pf);
+        case 2: return group_kernel_fn_g<2>(W, rg, pf);
+        case 4: return group_kernel_fn_g<4>(W, rg, pf);
+        case 8: return group_kernel_fn_g<8>(W, rg, pf);
+        case 16: return group_kernel_fn_g<16>(W, rg, pf);
+        case 32: return group_kernel_fn_g<32>(W, rg, pf);
+        case 64: return group_kernel_fn_g<64>(W, false, pf);
     }
     return nullptr;
 }
@@ -301,7 +314,8 @@ struct ctl_sim {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int n = 0, ns = 0, block = 256, grid = 0;
-    int lanes = 1;                   // lanes per simulation (1: tau_leap_kernel, else group_kernel<lanes>)
+    int lanes = 1;                   // lanes per simulation of the algorithm (1: tau_leap_kernel, else group_kernel<lanes, width>)
+    int width = 1;                   // lanes that execute one simulation (>= lanes)
     int compact = 0;                 // iterations between regroupings by mode (0: off)
     bool lds = false;
     size_t smem = 0;
@@ -539,17 +553,46 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         if ((size_t)gpb * gwords * 4 > 65536) gpb = 64 / G;   // one wavefront
         if ((size_t)gpb * gwords * 4 > 65536)
             return bail(ctl::fail(CTL_E_LIMIT, "model too large for this lanes_per_sim (use 64)"));
-        s->block = gpb * G;
+        // Lanes that execute a simulation.  When the simulations leave lanes
+        // of the chip empty, each takes W > G of them: the widest W at which
+        // all n are still resident at once (one more round of simulations
+        // costs more than the wider work gains).  Kernel times in ms, W = G /
+        // 16 / 32 / 64 (resident simulations at 16, 32, 64: 16384, 8192, 3072):
+        //   100x200 network, G = 16, t = 0.5   n =   24: - / 140 / 104 / 74
+        //                                      n = 4096: - / 156 / 118 / 152
+        //                                      n = 16384: - / 201 / 304 / -
+        //   50x100 network, G = 8, t = 0.2     n =  512: 188 / 125 / 80 / 67
+        //                                      n = 8192: 204 / 141 / 112 / 211
+        //                                      n = 32768: 248 / 358 / 413 / 756
+        //   enzyme cascade, G = 4, t = 50      n = 5003: 6.5 / 6.0 / 5.6 / 9.7
+        // At most 16 in force-SSA mode, whose steps are one chain of selection
+        // and update that a wider team does not shorten (cascade, n = 5003,
+        // force-SSA: 5.1 / 4.95 / 5.24 / 9.3).  An explicit geometry
+        // (block_size, slots, a regrouping interval) keeps W = G.
+        int W = G;
+        if (o->slots <= 0 && o->block_size <= 0 && o->compact_interval <= 0)
+            for (int w = o->force_ssa ? 16 : 64; w > G && w >= 16; w /= 2) {
+                const size_t sm = (size_t)(64 / w) * gwords * 4;
+                int cu = 0;
+                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&cu, group_kernel_fn(G, w, false, 1), 64, sm);
+                if (e == hipSuccess && (long long)prop.multiProcessorCount * cu * (64 / w) >= n) {
+                    W = w;
+                    gpb = 64 / w;                             // one wavefront per workgroup
+                    break;
+                }
+            }
+        s->width = W;
+        s->block = gpb * W;
         s->smem = (size_t)gpb * gwords * 4;
         s->lds = true;
-        s->compact = compact > 0 && G < 64 && s->block > 64 ? compact : 0;
-        const void* kfn = group_kernel_fn(G, s->compact > 0, 1);   // occupancy (the instances alike)
+        s->compact = compact > 0 && W == G && G < 64 && s->block > 64 ? compact : 0;
+        const void* kfn = group_kernel_fn(G, W, s->compact > 0, 1);   // occupancy (the instances alike)
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, s->block, s->smem);
         if (e != hipSuccess || per_cu <= 0) per_cu = 1;
         long long groups = o->slots > 0 ? (long long)o->slots : (long long)prop.multiProcessorCount * per_cu * gpb;
         if (groups > n) groups = ((n + gpb - 1) / gpb) * (long long)gpb;
         groups = ((groups + gpb - 1) / gpb) * gpb;
-        s->ns = (int)(groups * G);
+        s->ns = (int)(groups * W);
         s->grid = (int)(groups / gpb);
     } else {
         // regrouping slots by mode needs several wavefronts per workgroup
@@ -652,7 +695,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         p.oDp = put(Dptr.data(), Dptr.size());
         p.oDe = put(Dent.data(), Dent.size());
         p.oCs = put(reinterpret_cast<const uint32_t*>(m.cs.data()), m.cs.size());
-        if (s->lanes > 1) append_group_streams(T, p, s->lanes, m, FSptr, FSent, Dent);
+        if (s->lanes > 1) append_group_streams(T, p, s->lanes, s->width, m, FSptr, FSent, Dent);
         uint32_t* Td;
         if ((rc = upload(s, &Td, T.data(), T.size()))) return bail(rc);
         p.T = Td;
@@ -700,7 +743,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
     p.ns = ns;
     p.Cs = nullptr;
     if (G > 1) {                         // parked group state only: X [group][S]
-        if ((rc = dalloc(s, &p.X, (size_t)S * (ns / G))) || (rc = dalloc(s, &p.A, 1))) return bail(rc);
+        if ((rc = dalloc(s, &p.X, (size_t)S * (ns / s->width))) || (rc = dalloc(s, &p.A, 1))) return bail(rc);
     } else {
         if ((rc = dalloc(s, &p.X, (size_t)2 * S * ns)) || (rc = dalloc(s, &p.A, (size_t)R * ns))) return bail(rc);
         if (!p.c_bcast && (rc = dalloc(s, &p.Cs, (size_t)R * ns))) return bail(rc);
@@ -758,7 +801,7 @@ int ctl_sim_run(ctl_sim* s) {
                     hipLaunchKernelGGL(tau_leap_kernel<false>, dim3(s->grid), dim3(s->block), s->smem, s->stream, p);
                 break;
             default: {
-                const void* fn = group_kernel_fn(s->lanes, s->compact > 0, p.pfast);
+                const void* fn = group_kernel_fn(s->lanes, s->width, s->compact > 0, p.pfast);
                 if (!fn) return ctl::fail(CTL_E_STATE, "bad lanes_per_sim");
                 void* args[] = {&p};
                 HIPCHK(hipLaunchKernel(fn, dim3(s->grid), dim3(s->block), args, s->smem, s->stream),
