@@ -86,6 +86,10 @@ struct KParams {
     int pfast;                // propensity mode: 0 from the reactant entries; with <= 2 reactant entries of
                               //   multiplicity <= 2 per reaction (exactly 2 entries per round): 1 factor
                               //   indices into the LDS factor table, 2 entries read from the state
+    // Small models (small_kernel): words T[oST .. oST + nST), copied to LDS at
+    // the start of a launch (layout: ctl_small.h); nST = 0: not eligible.
+    int oST, nST, oSD;        // oSD: first word of the dependents in the table
+    int snf;                  // factor words per species (2, or 4 with a multiplicity of 3)
     const uint32_t* horw;     // hor | hort << 8
     const int32_t* cs;
     const double* ts;
@@ -113,6 +117,7 @@ struct KParams {
                               //   simulations by mode (0: never)
     // slots (global per-lane storage, [.][ns])
     int ns;
+    int lpw;                  // small_kernel: lanes of a wavefront that hold a slot
     int32_t* X;               // [2][S][ns]
     uint32_t* A;              // [R][ns]
     float* Cs;                // [R][ns] when rates differ between simulations
@@ -264,39 +269,10 @@ __device__ __forceinline__ void absorb(const KParams& p, Lane& L, const View& V,
     L.absorbed = 1;
 }
 
-// One adaptive leap attempt, PreCalculations (T.cu:1568-2093).
-__device__ __forceinline__ int leap(const KParams& p, Lane& L, const View& V, const float* __restrict__ recip) {
-    if (L.t >= p.tmax) return LEAP_DONE;
-    int32_t* X = xcur(V, L);
-    float a0c;
-    const float a0 = propensities(p, V, X, &a0c);
-    if (a0 == 0.0f) { absorb(p, L, V, X); return LEAP_ABSORB; }
-    // tau' over the species-major var flat (T.cu:1860-1922)
-    float tau1 = 3.40282347e+38f;
-    for (int sp = 0; sp < p.S; ++sp) {
-        const uint32_t h0 = CT_U32(p.Vptr)[sp], h1 = CT_U32(p.Vptr)[sp + 1];
-        if (h0 == h1) continue;
-        float mu = 0.0f, sg = 0.0f;
-        for (uint32_t h = h0; h < h1; ++h) {
-            const uint32_t e = CT_U32(p.Vent)[h];
-            const int j = (int)(e & 0xffffu);
-            const int v = (int)(int16_t)(e >> 16);
-            const uint32_t u = V.A[(size_t)j * V.st];
-            if (u & 0x80000000u) continue;
-            const float a = __uint_as_float(u);
-            mu = mu + (float)v * a;
-            sg = sg + (float)(v * v) * a;
-        }
-        if (mu == 0.0f || sg == 0.0f) continue;
-        const int32_t x = X[(size_t)sp * V.st];
-        const float gg = gfun(CT_U32(p.horw)[sp], x);
-        const float tmp2 = (p.eps * (float)x) / gg;
-        const float macs = tmp2 > 1.0f ? tmp2 : 1.0f;
-        const float t3 = macs / fabsf(mu);
-        const float t4 = (macs * macs) / sg;
-        const float tmp = t3 < t4 ? t3 : t4;
-        if (tmp < tau1) tau1 = tmp;
-    }
+// A leap attempt from tau' on (PreCalculations, T.cu:1935-2093): the switch
+// test, tau'' and the critical pick, the counts and the update, the samples.
+__device__ __forceinline__ int leap_from_tau(const KParams& p, Lane& L, const View& V, const float* __restrict__ recip,
+                                             int32_t* X, float tau1, float a0, float a0c) {
     if (tau1 < p.ssa_factor / a0) { L.switches++; return LEAP_SWITCH; }   // T.cu:1935-1941
     rng_event(L.g, L.evc++);
     float tau2 = 3.40282347e+38f;
@@ -395,6 +371,42 @@ __device__ __forceinline__ int leap(const KParams& p, Lane& L, const View& V, co
     L.firings += fired;
     L.leaps++;
     return LEAP_OK;
+}
+
+// One adaptive leap attempt, PreCalculations (T.cu:1568-2093).
+__device__ __forceinline__ int leap(const KParams& p, Lane& L, const View& V, const float* __restrict__ recip) {
+    if (L.t >= p.tmax) return LEAP_DONE;
+    int32_t* X = xcur(V, L);
+    float a0c;
+    const float a0 = propensities(p, V, X, &a0c);
+    if (a0 == 0.0f) { absorb(p, L, V, X); return LEAP_ABSORB; }
+    // tau' over the species-major var flat (T.cu:1860-1922)
+    float tau1 = 3.40282347e+38f;
+    for (int sp = 0; sp < p.S; ++sp) {
+        const uint32_t h0 = CT_U32(p.Vptr)[sp], h1 = CT_U32(p.Vptr)[sp + 1];
+        if (h0 == h1) continue;
+        float mu = 0.0f, sg = 0.0f;
+        for (uint32_t h = h0; h < h1; ++h) {
+            const uint32_t e = CT_U32(p.Vent)[h];
+            const int j = (int)(e & 0xffffu);
+            const int v = (int)(int16_t)(e >> 16);
+            const uint32_t u = V.A[(size_t)j * V.st];
+            if (u & 0x80000000u) continue;
+            const float a = __uint_as_float(u);
+            mu = mu + (float)v * a;
+            sg = sg + (float)(v * v) * a;
+        }
+        if (mu == 0.0f || sg == 0.0f) continue;
+        const int32_t x = X[(size_t)sp * V.st];
+        const float gg = gfun(CT_U32(p.horw)[sp], x);
+        const float tmp2 = (p.eps * (float)x) / gg;
+        const float macs = tmp2 > 1.0f ? tmp2 : 1.0f;
+        const float t3 = macs / fabsf(mu);
+        const float t4 = (macs * macs) / sg;
+        const float tmp = t3 < t4 ? t3 : t4;
+        if (tmp < tau1) tau1 = tmp;
+    }
+    return leap_from_tau(p, L, V, recip, X, tau1, a0, a0c);
 }
 
 // Up to `steps` direct-method SSA steps of the current burst

@@ -30,11 +30,13 @@
 #include "ctl_group.h"
 #include "ctl_internal.h"
 #include "ctl_kernels.h"
+#include "ctl_small.h"
 
 #pragma clang fp contract(off)
 
 namespace ctl {
 
+// The one-lane kernel (ctl_small.h runs the default geometry of small models).
 // One slot per lane; kLDS keeps the lane's state, trial state, propensities
 // (and per-simulation rates) in LDS for the duration of the launch, copied
 // from / to the global slot arrays at entry / exit.  With p.compact > 0 (and
@@ -138,6 +140,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
         L.xb = 0;
     }
     store_lane(p, L);
+}
+
+const void* small_kernel_fn(int R) {
+    return small_batch(R) == 4 ? (const void*)small_kernel<4> : (const void*)small_kernel<8>;
 }
 
 // The group kernel instance for the G-lane algorithm on W lanes per
@@ -316,6 +322,8 @@ struct ctl_sim {
     int n = 0, ns = 0, block = 256, grid = 0;
     int lanes = 1;                   // lanes per simulation of the algorithm (1: tau_leap_kernel, else group_kernel<lanes, width>)
     int width = 1;                   // lanes that execute one simulation (>= lanes)
+    bool small = false;              // one lane per simulation: small_kernel
+    int lpw = 64;                    // one lane per simulation: lanes of a workgroup that hold one
     int compact = 0;                 // iterations between regroupings by mode (0: off)
     bool lds = false;
     size_t smem = 0;
@@ -512,6 +520,26 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
     e = hipGetDeviceProperties(&prop, s->device);
     if (e != hipSuccess) return bail(hip_fail(e, "hipGetDeviceProperties"));
     const int S = m.S, R = m.R, K = (int)m.ts.size(), SS = (int)m.cs.size();
+    // SSA dependency graph: for each reaction j, the reactions with a
+    // reactant among the species j changes (its fear entries), ascending.
+    std::vector<uint32_t> Dptr(R + 1, 0), Dent;
+    {
+        std::vector<std::vector<uint32_t>> readers(S);
+        for (int r = 0; r < R; ++r)
+            for (uint32_t h = m.Lptr[r]; h < m.Lptr[r + 1]; ++h) readers[m.Lent[h] & 0xffffu].push_back((uint32_t)r);
+        std::vector<char> mark(R, 0);
+        std::vector<uint32_t> list;
+        for (int j = 0; j < R; ++j) {
+            Dptr[j] = (uint32_t)Dent.size();
+            list.clear();
+            for (uint32_t h = m.Fptr[j]; h < m.Fptr[j + 1]; ++h)
+                for (uint32_t r : readers[m.Fent[h] & 0xffffu])
+                    if (!mark[r]) { mark[r] = 1; list.push_back(r); }
+            std::sort(list.begin(), list.end());
+            for (uint32_t r : list) { mark[r] = 0; Dent.push_back(r); }
+        }
+        Dptr[R] = (uint32_t)Dent.size();
+    }
     // Launch geometry.  One lane per simulation when its working set (state,
     // trial state, propensities, per-simulation rates) fits a 64-lane
     // wavefront's 16 KB share of LDS, or when asked for; otherwise G lanes
@@ -532,6 +560,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         return bail(ctl::fail(CTL_E_ARGS, "lanes_per_sim must be 0 or a power of two up to 64"));
     s->lanes = G;
     int per_cu = 0;
+    std::vector<uint32_t> small_tab;         // small_kernel's table (empty: not used)
     if (G > 1) {
         const size_t gwords = group_lds_words(S, R, G);    // group LDS words per simulation
         if (gwords * 4 > 65536) return bail(ctl::fail(CTL_E_LIMIT, "model too large for the group kernel (more than 64 KB of LDS)"));
@@ -616,14 +645,39 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
             s->smem = smem_of(false, s->block);
         }
         s->compact = compact > 0 && s->block > 64 ? compact : 0;
-        const void* kfn = s->lds ? (const void*)tau_leap_kernel<true> : (const void*)tau_leap_kernel<false>;
+        // The default geometry of an LDS model runs small_kernel where the model
+        // is eligible; an explicit workgroup size or regrouping interval runs
+        // tau_leap_kernel.
+        s->lpw = s->block;
+        if (s->lds && o->block_size == 0 && compact <= 0 && o->nc < (1 << 24)) {
+            small_tab = small_table(m, Dptr, Dent, &s->kp.oSD, &s->kp.snf);
+            if (!small_tab.empty()) {
+                s->small = true;
+                s->smem = (small_tab.size() + (m.c_rows == 1 ? R : 0)) * 4 +
+                          (size_t)small_words(S, R, s->kp.snf, m.c_rows == 1) * 4 * 64;
+                // Lanes of a wavefront that hold a simulation: 64 when the
+                // simulations fill the chip, and in force-SSA mode, where the
+                // lanes of a wavefront run in step; adaptive runs with up to
+                // two simulations per resident wavefront spread out, since
+                // leaps and SSA bursts of one wavefront's lanes run one after
+                // the other.  Schlogl to t = 10, kernel ms at 1 / 2 / 8 / 64
+                // lanes: n = 1024 52 / 60 / 62 / 79, n = 4096 56 / 62 / 76 /
+                // 81; to t = 2.5, n = 16384 (8 / 64) 21.3 / 21.0; force-SSA to
+                // t = 1, n = 4096: 9.7 / 8.4 / 8.6 / 7.7.
+                const long long waves = (long long)prop.multiProcessorCount * 16;
+                if (!o->force_ssa && o->slots <= 0 && n <= 2 * waves) s->lpw = n <= waves ? 1 : 2;
+                s->smem = (small_tab.size() + (m.c_rows == 1 ? R : 0)) * 4 +
+                          (size_t)small_words(S, R, s->kp.snf, m.c_rows == 1) * 4 * s->lpw;
+            }
+        }
+        const void* kfn = s->small ? small_kernel_fn(R) : s->lds ? (const void*)tau_leap_kernel<true> : (const void*)tau_leap_kernel<false>;
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, s->block, s->smem);
         if (e != hipSuccess || per_cu <= 0) per_cu = 1;
-        int ns = o->slots > 0 ? o->slots : prop.multiProcessorCount * per_cu * s->block;
-        if (ns > n) ns = ((n + s->block - 1) / s->block) * s->block;
-        if (s->compact) ns = ((ns + s->block - 1) / s->block) * s->block;   // whole workgroups
+        int ns = o->slots > 0 ? o->slots : prop.multiProcessorCount * per_cu * s->lpw;
+        if (ns > n) ns = ((n + s->lpw - 1) / s->lpw) * s->lpw;
+        if (s->compact) ns = ((ns + s->lpw - 1) / s->lpw) * s->lpw;   // whole workgroups
         s->ns = ns;
-        s->grid = (ns + s->block - 1) / s->block;
+        s->grid = (ns + s->lpw - 1) / s->lpw;
     }
     const int ns = s->ns;
 
@@ -634,26 +688,6 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
     for (int i = 0; i < S; ++i) horw[i] = (uint32_t)m.hor[i] | ((uint32_t)m.hort[i] << 8);
     std::vector<float> cf(m.c.size());
     for (size_t i = 0; i < m.c.size(); ++i) cf[i] = (float)m.c[i];
-    // SSA dependency graph: for each reaction j, the reactions with a
-    // reactant among the species j changes (its fear entries), ascending.
-    std::vector<uint32_t> Dptr(R + 1, 0), Dent;
-    {
-        std::vector<std::vector<uint32_t>> readers(S);
-        for (int r = 0; r < R; ++r)
-            for (uint32_t h = m.Lptr[r]; h < m.Lptr[r + 1]; ++h) readers[m.Lent[h] & 0xffffu].push_back((uint32_t)r);
-        std::vector<char> mark(R, 0);
-        std::vector<uint32_t> list;
-        for (int j = 0; j < R; ++j) {
-            Dptr[j] = (uint32_t)Dent.size();
-            list.clear();
-            for (uint32_t h = m.Fptr[j]; h < m.Fptr[j + 1]; ++h)
-                for (uint32_t r : readers[m.Fent[h] & 0xffffu])
-                    if (!mark[r]) { mark[r] = 1; list.push_back(r); }
-            std::sort(list.begin(), list.end());
-            for (uint32_t r : list) { mark[r] = 0; Dent.push_back(r); }
-        }
-        Dptr[R] = (uint32_t)Dent.size();
-    }
     // fear entries species-major, ascending reaction (group kernel update)
     std::vector<uint32_t> FSptr(S + 1, 0), FSent(m.Fent.size());
     {
@@ -696,6 +730,8 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         p.oDe = put(Dent.data(), Dent.size());
         p.oCs = put(reinterpret_cast<const uint32_t*>(m.cs.data()), m.cs.size());
         if (s->lanes > 1) append_group_streams(T, p, s->lanes, s->width, m, FSptr, FSent, Dent);
+        p.oST = put(small_tab.data(), small_tab.size());
+        p.nST = (int)small_tab.size();
         uint32_t* Td;
         if ((rc = upload(s, &Td, T.data(), T.size()))) return bail(rc);
         p.T = Td;
@@ -741,6 +777,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
     p.compact = s->compact;
     p.iters = o->iters_per_launch > 0 ? o->iters_per_launch : (G > 1 ? 65536 : 4096);
     p.ns = ns;
+    p.lpw = s->lpw;
     p.Cs = nullptr;
     if (G > 1) {                         // parked group state only: X [group][S]
         if ((rc = dalloc(s, &p.X, (size_t)S * (ns / s->width))) || (rc = dalloc(s, &p.A, 1))) return bail(rc);
@@ -795,7 +832,11 @@ int ctl_sim_run(ctl_sim* s) {
         HIPCHK(hipEventRecord(s->ev0, s->stream), "hipEventRecord");
         switch (s->lanes) {
             case 1:
-                if (s->lds)
+                if (s->small) {
+                    void* args[] = {&p};
+                    HIPCHK(hipLaunchKernel(small_kernel_fn(p.R), dim3(s->grid), dim3(64), args, s->smem, s->stream),
+                           "small_kernel launch");
+                } else if (s->lds)
                     hipLaunchKernelGGL(tau_leap_kernel<true>, dim3(s->grid), dim3(s->block), s->smem, s->stream, p);
                 else
                     hipLaunchKernelGGL(tau_leap_kernel<false>, dim3(s->grid), dim3(s->block), s->smem, s->stream, p);
