@@ -331,7 +331,7 @@ int upload_model(ctl_batch* b, const ctl::Model& m, KParams& p, int G, int W) {
         p.oDp = put(Dptr.data(), Dptr.size());
         p.oDe = put(Dent.data(), Dent.size());
         p.oCs = put(reinterpret_cast<const uint32_t*>(m.cs.data()), m.cs.size());
-        if (G > 1) append_group_streams(T, p, G, W, m, FSptr, FSent, Dent);
+        if (G > 1) append_group_streams(T, p, G, W, m, FSptr, FSent, Dptr, Dent);
         uint32_t* Td;
         if ((rc = bupload(b, &Td, T.data(), T.size()))) return rc;
         p.T = Td;

@@ -345,6 +345,24 @@ __device__ __forceinline__ uint32_t grng_u32(GRng& g, int l) {
     return __shfl(mine, src, W);
 }
 
+// Two consecutive words of one block (an SSA step's: an event's steps consume
+// two words each, so a pair never spans blocks).
+template <int W>
+__device__ __forceinline__ void grng_pair(GRng& g, int l, uint32_t& w0, uint32_t& w1) {
+    const uint32_t b = g.wc >> 2;
+    if (b - g.cb >= (uint32_t)W) {
+        g.cb = b;
+        philox_block(b + (uint32_t)l, g.ev, g.sim, 0u, g.k0, g.k1, g.c0, g.c1, g.c2, g.c3);
+    }
+    uint32_t c0 = g.c0, c1 = g.c1, c2 = g.c2, c3 = g.c3;      // values: see grng_u32
+    asm volatile("" : "+v"(c0), "+v"(c1), "+v"(c2), "+v"(c3));
+    const bool hi = (g.wc & 2u) != 0u;
+    const int src = (int)(b - g.cb);
+    g.wc += 2u;
+    w0 = __shfl(hi ? c2 : c0, src, W);
+    w1 = __shfl(hi ? c3 : c1, src, W);
+}
+
 struct GLane {
     int slot;                // group slot
     int sim;                 // local index, -1 none, -2 queue exhausted
@@ -659,7 +677,7 @@ __device__ __forceinline__ void gprops(const KParams& p, const int32_t* X, const
 // so such a lane's inclusive sum can round above its predecessor's.  Only a
 // reaction with a positive propensity is chosen.  Returns the chosen
 // reaction (group-uniform) or -1 when no lane has a positive partial.
-template <int G>
+template <int G, int W>
 __device__ __forceinline__ int gselect(const KParams& p, const uint32_t* A, float Pown, float P, float w, int l,
                                        int which) {
     const uint64_t cand = gballot<G>(Pown > 0.0f);
@@ -668,20 +686,20 @@ __device__ __forceinline__ int gselect(const KParams& p, const uint32_t* A, floa
     const int sel = hit ? __builtin_ctzll(hit) : 63 - __builtin_clzll(cand);
     const float excl = G <= 16 ? dppf<DPP_ROW_SHR1>(P) : dppf<DPP_WAVE_SHR1>(P);   // lane 0's value is unused
     // The walk through lane sel's reactions sel + i*G, spread over the first
-    // W lanes of the group (a row of 16 at most): lane i holds the i-th
+    // N lanes of the team (a row of 16 at most): lane i holds the i-th
     // propensity and the sequential sums excl + a_0 + ... + a_i are built by
-    // W-1 row shifts (after k shifts lanes 0..k hold their final sum; a
+    // N-1 row shifts (after k shifts lanes 0..k hold their final sum; a
     // shifted-in 0 or a skipped entry adds an exact 0), so every sum is
     // rounded as in the one-lane walk.  Lane sel's reactions number at most
-    // 16 per round; groups wider than 16 leave their other rows idle.
-    constexpr int W = G <= 16 ? G : 16;
+    // 16 per round; wider teams leave their other rows idle.
+    constexpr int N = W <= 16 ? W : 16;
     const int nj = (p.R - sel + G - 1) / G;
     float carry = __shfl(excl, sel, G);
     if (sel == 0) carry = 0.0f;
     int last = -1;
-    for (int c = 0; c < nj; c += W) {
+    for (int c = 0; c < nj; c += N) {
         const int i = c + l;
-        const bool in = l < W && i < nj;
+        const bool in = l < N && i < nj;
         const int j = sel + i * G;
         const uint32_t u = in ? A[j] : 0u;
         const bool use = which != 2 || (u & 0x80000000u) || j == 0;
@@ -689,17 +707,55 @@ __device__ __forceinline__ int gselect(const KParams& p, const uint32_t* A, floa
         const float a1 = l == 0 ? carry + a : a;
         float x = a1;
 #pragma unroll
-        for (int k = 1; k < W; ++k) {
+        for (int k = 1; k < N; ++k) {
             const float t = dppf<DPP_ROW_SHR1>(x) + a1;
-            x = (W == 16 || l > 0) ? t : a1;
+            x = (N == 16 || l > 0) ? t : a1;
         }
-        const uint64_t pos = gballot<G>(in && a > 0.0f);
-        const uint64_t hm = gballot<G>(in && a > 0.0f && w <= x);
+        const uint64_t pos = gballot<W>(in && a > 0.0f);
+        const uint64_t hm = gballot<W>(in && a > 0.0f && w <= x);
         if (hm) return sel + (c + __builtin_ctzll(hm)) * G;
         if (pos) last = sel + (c + 63 - __builtin_clzll(pos)) * G;
-        carry = G <= 16 ? gbcast_last<G>(x, l) : __shfl(x, W - 1, G);
+        carry = W <= 16 ? gbcast_last<W>(x, l) : __shfl(x, N - 1, W);
     }
     return last;
+}
+
+// gselect over all reactions with the walk done by every lane of the group
+// alike: the chosen lane's propensities are read in batches of eight and
+// summed from its predecessor's inclusive sum, as the one-lane walk does.
+// More instructions than a round of the fold, so it pays only where the fold
+// has two lanes to spread over (50x100 network, G = 2, 65536 simulations: 1640
+// ms with the fold, 1414 with the walk; enzyme cascade, G = 4: 23.6 and 28.9).
+template <int G>
+__device__ __forceinline__ int gselect_walk(const KParams& p, const uint32_t* A, float Pown, float P, float w, int l) {
+    const uint64_t cand = gballot<G>(Pown > 0.0f);
+    if (cand == 0) return -1;
+    const uint64_t hit = gballot<G>(Pown > 0.0f && P >= w);
+    const int sel = hit ? __builtin_ctzll(hit) : 63 - __builtin_clzll(cand);
+    const float excl = G <= 16 ? dppf<DPP_ROW_SHR1>(P) : dppf<DPP_WAVE_SHR1>(P);   // lane 0's value is unused
+    float x = __shfl(excl, sel, G);
+    if (sel == 0) x = 0.0f;
+    const int nrp = group_rpad(p.R, G) / G;
+    int first = -1, last = -1;
+    for (int c = 0; c < nrp; c += 8) {
+        uint32_t u[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) u[i] = A[sel + (c + i < nrp ? c + i : nrp - 1) * G];
+        int f = -1;
+        float xs[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (c + i >= nrp) u[i] = 0u;                       // past the padding
+            x = x + aval(u[i]);
+            xs[i] = x;
+        }
+#pragma unroll
+        for (int i = 7; i >= 0; --i) f = aval(u[i]) > 0.0f && w <= xs[i] ? c + i : f;
+        first = first < 0 ? f : first;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) last = aval(u[i]) > 0.0f ? c + i : last;
+    }
+    return sel + (first >= 0 ? first : last) * G;
 }
 
 template <int W>
@@ -820,7 +876,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         }
         const float Qown = Q;
         Q = gscan<G>(Q, la);
-        pick = gselect<G>(p, V.A, Qown, Q, w, la, 2);
+        pick = gselect<G, W>(p, V.A, Qown, Q, w, l, 2);
     }
     CTL_PHASE(PH_PICK);
     uint64_t fired = 0;
@@ -965,6 +1021,19 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
     return LEAP_OK;
 }
 
+// The sampled species of state X to row (four reads in flight).
+template <int W>
+__device__ __forceinline__ void gsample(const KParams& p, const int32_t* X, uint32_t* row, int l) {
+    for (int s0 = l; s0 < p.SS; s0 += 4 * W) {
+        uint32_t sp[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sp[i] = p.T[p.oCs + (s0 + i * W < p.SS ? s0 + i * W : s0)];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (s0 + i * W < p.SS) row[s0 + i * W] = (uint32_t)X[sp[i]];
+    }
+}
+
 // Up to nmax steps of an SSA burst (EventualSSASteps T.cu:2099-2273 /
 // LightweightSSA T.cu:2280-2454), opening the burst when none is in progress:
 // a burst of p.ssa_steps steps may run in several calls, its clock advance,
@@ -991,6 +1060,11 @@ __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView
     CTL_PHASE(PH_SSA_OPEN);
     double tacc = L.tacc;
     const int n = nmax < L.ssa_left ? nmax : L.ssa_left;
+    const int pm = pmode<PFM>(kuse(p.pfast));
+    const bool fac = pm == 1;
+    const uint4* SR = reinterpret_cast<const uint4*>(p.T + p.oSR);
+    const uint4* DR = reinterpret_cast<const uint4*>(p.T + p.oDR);
+    double tnext = L.cursor < (uint32_t)p.K ? p.ts[L.cursor] : 0.0;        // the next sample time
     for (int step = 0; step < n; ++step) {
         float P = 0.0f;
         const int nrp = group_rpad(p.R, G) / G;        // rounds over A with its zero padding
@@ -1005,66 +1079,68 @@ __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView
         P = gscan<G>(P, la);
         const float a0 = gbcast_last<G>(P, la);
         if (a0 == 0.0f) { gabsorb<W>(p, L, X, l); L.ssa_left = 0; return true; }
-        const float r1 = u32_oc(grng_u32<W>(L.gg, l)) * a0;
-        const int j = gselect<G>(p, V.A, Pown, P, r1, la, 0);
+        uint32_t w0, w1;
+        grng_pair<W>(L.gg, l, w0, w1);
+        const float r1 = u32_oc(w0) * a0;
+        const int j = W < 4 ? gselect_walk<G>(p, V.A, Pown, P, r1, la) : gselect<G, W>(p, V.A, Pown, P, r1, l, 0);
         if (j < 0) { gabsorb<W>(p, L, X, l); L.ssa_left = 0; return true; }    // unreachable for finite a0
-        const float dt = u32_exp(grng_u32<W>(L.gg, l)) / a0;
+        const uint4 sr = SR[j];              // {first change entry, count, first dependent, count}
+        const float dt = u32_exp(w1) / a0;
         CTL_PHASE(PH_SSA_SELECT);
         tacc = tacc + (double)dt;
         const double tn = L.t + tacc;
-        uint32_t i = L.cursor;
-        if (i < (uint32_t)p.K && tn > p.ts[i]) {                               // T.cu:2213-2236
+        // this lane's first change entry and dependent: one latency for both
+        uint32_t ent = 0u;
+        uint4 rec = make_uint4(0u, 0u, 0u, 0u);
+        const bool hasf = (uint32_t)l < sr.y, hasd = (uint32_t)l < sr.w;
+        if (hasf) ent = p.T[sr.x + (uint32_t)l];
+        if (pm != 0 && hasd) rec = DR[sr.z + (uint32_t)l];
+        if (L.cursor < (uint32_t)p.K && tn > tnext) {                          // T.cu:2213-2236
+            uint32_t i = L.cursor;
             uint32_t* out = p.storage + (size_t)L.sim * p.K * p.SS;
             while (i < (uint32_t)p.K && tn > p.ts[i]) {
-                for (int sk = l; sk < p.SS; sk += W) out[(size_t)i * p.SS + sk] = (uint32_t)X[p.T[p.oCs + sk]];
+                gsample<W>(p, X, out + (size_t)i * p.SS, l);
                 ++i;
             }
             L.cursor = i;
+            tnext = i < (uint32_t)p.K ? p.ts[i] : 0.0;
+            gsync();
         }
-        gsync();
-        const uint32_t f1 = p.T[p.oFp + j + 1];
-        const int pm = pmode<PFM>(kuse(p.pfast));
-        const bool fac = pm == 1;
-        for (uint32_t h = p.T[p.oFp + j] + (uint32_t)l; h < f1; h += W) {
-            const uint32_t ent = p.T[p.oFe + h];
-            const int s = (int)(ent & 0xffffu);
-            const int v = (int)(int16_t)(ent >> 16);
-            const int32_t x = (int32_t)((uint32_t)X[s] + (uint32_t)v);
+        float c = 0.0f;
+        if (pm != 0 && hasd) c = p.drate ? __uint_as_float(rec.w) : L.crate[rec.x];
+        auto change = [&](uint32_t e) {      // a species occurs once per reaction
+            const int s = (int)(e & 0xffffu);
+            const int32_t x = (int32_t)((uint32_t)X[s] + (uint32_t)(int)(int16_t)(e >> 16));
             X[s] = x;
-            if (fac) gfactor(V.F, p.S, s, x, (uint32_t)p.nc);   // a species occurs once per reaction
-        }
+            if (fac) gfactor(V.F, p.S, s, x, (uint32_t)p.nc);
+        };
+        if (hasf) change(ent);
+        for (uint32_t h = (uint32_t)l + W; h < sr.y; h += W) change(p.T[sr.x + h]);
         gsync();
         CTL_PHASE(PH_SSA_UPDATE);
         L.ssa_steps++;
         if (tn <= p.tmax) L.firings++;
-        const uint32_t d0 = p.T[p.oDp + j], d1 = p.T[p.oDp + j + 1];
-        if (fac) {
-            // dependent records {r, factor index 0, factor index 1, 0}: one 16-byte load each
-            const uint4* DR = reinterpret_cast<const uint4*>(p.T + p.oDR);
-            for (uint32_t d = d0 + (uint32_t)l; d < d1; d += W) {
-                const uint4 rec = DR[d];
-                const int r = (int)rec.x;
-                const uint32_t u0 = V.F[rec.y], u1 = V.F[rec.z];
-                float a = L.crate[r];
-                a = a * __uint_as_float(u0 & 0x7fffffffu);
-                a = a * __uint_as_float(u1 & 0x7fffffffu);
-                V.A[r] = __float_as_uint(a) | ((u0 | u1) & 0x80000000u);
-            }
-        } else if (pm == 2) {
-            // dependent records {r, reactant entry 0, entry 1, 0} read from the state
-            const uint4* DR = reinterpret_cast<const uint4*>(p.T + p.oDR);
-            const uint32_t nc = (uint32_t)p.nc;
-            for (uint32_t d = d0 + (uint32_t)l; d < d1; d += W) {
-                const uint4 rec = DR[d];
-                const int r = (int)rec.x;
-                float a = L.crate[r];
-                bool c = false;
-                gtwo(a, c, X[rec.y & 0xffffu], rec.y >> 16, X[rec.z & 0xffffu], rec.z >> 16, nc);
-                V.A[r] = __float_as_uint(a) | (c ? 0x80000000u : 0u);
+        if (pm != 0) {
+            auto depend = [&](const uint4& d, float a) {
+                if (fac) {                   // {r, factor index 0, factor index 1, rate}
+                    const uint32_t u0 = V.F[d.y], u1 = V.F[d.z];
+                    a = a * __uint_as_float(u0 & 0x7fffffffu);
+                    a = a * __uint_as_float(u1 & 0x7fffffffu);
+                    V.A[d.x] = __float_as_uint(a) | ((u0 | u1) & 0x80000000u);
+                } else {                     // {r, reactant entry 0, entry 1, rate} read from the state
+                    bool crit = false;
+                    gtwo(a, crit, X[d.y & 0xffffu], d.y >> 16, X[d.z & 0xffffu], d.z >> 16, (uint32_t)p.nc);
+                    V.A[d.x] = __float_as_uint(a) | (crit ? 0x80000000u : 0u);
+                }
+            };
+            if (hasd) depend(rec, c);
+            for (uint32_t d = (uint32_t)l + W; d < sr.w; d += W) {
+                const uint4 q = DR[sr.z + d];
+                depend(q, p.drate ? __uint_as_float(q.w) : L.crate[q.x]);
             }
         } else {
-            for (uint32_t d = d0 + (uint32_t)l; d < d1; d += W) {
-                const int r = (int)p.T[p.oDe + d];
+            for (uint32_t d = (uint32_t)l; d < sr.w; d += W) {
+                const int r = (int)p.T[p.oDe + sr.z + d];
                 bool crit;
                 const float a = gprop(p, X, L.crate, r, crit);
                 V.A[r] = __float_as_uint(a) | (crit ? 0x80000000u : 0u);
@@ -1438,7 +1514,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gwaves(G, W
 // group kernel with G lanes to the packed table buffer T.
 inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, int W, const Model& m,
                                  const std::vector<uint32_t>& FSptr, const std::vector<uint32_t>& FSent,
-                                 const std::vector<uint32_t>& Dent) {
+                                 const std::vector<uint32_t>& Dptr, const std::vector<uint32_t>& Dent) {
     // Item order[r * B + l] (-1: none) goes to lane l of round r of B lanes.  fixed > 0:
     // every round has exactly that many entries per lane; else the round's
     // longest list rounded up to a multiple of quantum.
@@ -1492,9 +1568,17 @@ inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, in
     } else {
         rounds(G, rorder, m.Lptr, m.Lent, p.oPRm, p.oPRe, 1, p.pfast == 2 ? 2 : 0, 0u);
     }
-    p.oDR = 0;
-    if (p.pfast) {                        // dependent records, 16-byte aligned
-        while (T.size() % 4) T.push_back(0u);
+    while (T.size() % 4) T.push_back(0u);   // per reaction {first change entry, count, first dependent, count}
+    p.oSR = (int)T.size();
+    for (int j = 0; j < m.R; ++j) {
+        T.push_back((uint32_t)p.oFe + m.Fptr[j]);
+        T.push_back(m.Fptr[j + 1] - m.Fptr[j]);
+        T.push_back(Dptr[j]);
+        T.push_back(Dptr[j + 1] - Dptr[j]);
+    }
+    p.oDR = p.oSR;
+    p.drate = m.c_rows == 1;
+    if (p.pfast) {                        // dependent records
         p.oDR = (int)T.size();
         for (uint32_t r : Dent) {       // factor indices (mode 1) or the entries themselves (mode 2)
             const uint32_t n = m.Lptr[r + 1] - m.Lptr[r];
@@ -1502,7 +1586,7 @@ inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, in
             T.push_back(r);
             T.push_back(p.pfast == 1 ? (n > 0 ? findex(e0) : one) : e0);
             T.push_back(p.pfast == 1 ? (n > 1 ? findex(e1) : one) : e1);
-            T.push_back(0u);
+            T.push_back(p.drate ? __builtin_bit_cast(uint32_t, (float)m.c[r]) : 0u);
         }
     }
     // species by entry count, longest first, so that a round's lanes carry

@@ -593,10 +593,10 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         //   50x100 network, G = 8, t = 0.2     n =  512: 188 / 125 / 80 / 67
         //                                      n = 8192: 204 / 141 / 112 / 211
         //                                      n = 32768: 248 / 358 / 413 / 756
-        //   enzyme cascade, G = 4, t = 50      n = 5003: 6.5 / 6.0 / 5.6 / 9.7
-        // At most 16 in force-SSA mode, whose steps are one chain of selection
-        // and update that a wider team does not shorten (cascade, n = 5003,
-        // force-SSA: 5.1 / 4.95 / 5.24 / 9.3).  An explicit geometry
+        //   enzyme cascade, G = 4, t = 50      n = 5003: 6.2 / 5.4 / 5.2 / 5.3
+        // At most 16 in force-SSA mode: an SSA step is one chain of selection
+        // and update that a wider team does not shorten (cascade of 13 stages,
+        // n = 5003, force-SSA: 4.8 / 4.6 / 5.0 / 5.1).  An explicit geometry
         // (block_size, slots, a regrouping interval) keeps W = G.
         int W = G;
         if (o->slots <= 0 && o->block_size <= 0 && o->compact_interval <= 0)
@@ -729,7 +729,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         p.oDp = put(Dptr.data(), Dptr.size());
         p.oDe = put(Dent.data(), Dent.size());
         p.oCs = put(reinterpret_cast<const uint32_t*>(m.cs.data()), m.cs.size());
-        if (s->lanes > 1) append_group_streams(T, p, s->lanes, s->width, m, FSptr, FSent, Dent);
+        if (s->lanes > 1) append_group_streams(T, p, s->lanes, s->width, m, FSptr, FSent, Dptr, Dent);
         p.oST = put(small_tab.data(), small_tab.size());
         p.nST = (int)small_tab.size();
         uint32_t* Td;
