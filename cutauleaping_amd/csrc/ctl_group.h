@@ -720,42 +720,81 @@ __device__ __forceinline__ int gselect(const KParams& p, const uint32_t* A, floa
     return last;
 }
 
-// gselect over all reactions with the walk done by every lane of the group
-// alike: the chosen lane's propensities are read in batches of eight and
-// summed from its predecessor's inclusive sum, as the one-lane walk does.
-// More instructions than a round of the fold, so it pays only where the fold
-// has two lanes to spread over (50x100 network, G = 2, 65536 simulations: 1640
-// ms with the fold, 1414 with the walk; enzyme cascade, G = 4: 23.6 and 28.9).
-template <int G>
-__device__ __forceinline__ int gselect_walk(const KParams& p, const uint32_t* A, float Pown, float P, float w, int l) {
-    const uint64_t cand = gballot<G>(Pown > 0.0f);
-    if (cand == 0) return -1;
+// Minimum of an int over N lanes (N <= 16).
+template <int N>
+__device__ __forceinline__ int gmini(int v) {
+    auto step = [&](int o) { v = o < v ? o : v; };
+    if (N >= 2) step(__builtin_amdgcn_update_dpp(v, v, DPP_QP_1032, 0xf, 0xf, false));
+    if (N >= 4) step(__builtin_amdgcn_update_dpp(v, v, DPP_QP_2301, 0xf, 0xf, false));
+    if (N >= 8) step(__builtin_amdgcn_update_dpp(v, v, DPP_ROW_HALF_MIRROR, 0xf, 0xf, false));
+    if (N >= 16) step(__builtin_amdgcn_update_dpp(v, v, DPP_ROW_MIRROR, 0xf, 0xf, false));
+    return v;
+}
+
+// gselect over all reactions (which = 0) for the SSA step, without branches
+// that depend on the simulation: a taken branch costs about 20 ns, and
+// straight-line code lets the step's exponential run between the row shifts.
+// cand: the lanes with a positive partial (not 0).  Teams narrower than 16
+// fold in chunks of N reactions, each lane keeping the first of its own that
+// reaches w.
+template <int G, int W>
+__device__ __forceinline__ int gselect_ssa(const uint32_t* A, uint64_t cand, float Pown, float P, float w, int l,
+                                           int nrp) {
     const uint64_t hit = gballot<G>(Pown > 0.0f && P >= w);
     const int sel = hit ? __builtin_ctzll(hit) : 63 - __builtin_clzll(cand);
     const float excl = G <= 16 ? dppf<DPP_ROW_SHR1>(P) : dppf<DPP_WAVE_SHR1>(P);   // lane 0's value is unused
-    float x = __shfl(excl, sel, G);
-    if (sel == 0) x = 0.0f;
-    const int nrp = group_rpad(p.R, G) / G;
-    int first = -1, last = -1;
-    for (int c = 0; c < nrp; c += 8) {
-        uint32_t u[8];
+    constexpr int N = W <= 16 ? W : 16;
+    float carry = __shfl(excl, sel, G);
+    if (sel == 0) carry = 0.0f;
+    if (N == 16 && nrp <= 16) {              // the usual case: at most 16 reactions per lane
+        const uint32_t u = A[sel + (l < nrp ? l : 0) * G];
+        const float a = l < nrp ? aval(u) : 0.0f;
+        const float a1 = l == 0 ? carry + a : a;
+        float x = a1;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) u[i] = A[sel + (c + i < nrp ? c + i : nrp - 1) * G];
-        int f = -1;
-        float xs[8];
+        for (int k = 1; k < 16; ++k) x = dppf<DPP_ROW_SHR1>(x) + a1;
+        const uint64_t pos = gballot<W>(l < 16 && a > 0.0f);
+        const uint64_t hm = gballot<W>(l < 16 && a > 0.0f && w <= x);
+        return sel + (hm ? __builtin_ctzll(hm) : 63 - __builtin_clzll(pos)) * G;
+    }
+    constexpr int NONE = 0x7fffffff;
+    int first = NONE;
+    for (int c0 = 0; c0 < nrp; c0 += 4 * N) {
+        uint32_t u[4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            if (c + i >= nrp) u[i] = 0u;                       // past the padding
-            x = x + aval(u[i]);
-            xs[i] = x;
+        for (int q = 0; q < 4; ++q) {
+            const int i = c0 + q * N + l;
+            u[q] = A[sel + (i < nrp ? i : nrp - 1) * G];
         }
 #pragma unroll
-        for (int i = 7; i >= 0; --i) f = aval(u[i]) > 0.0f && w <= xs[i] ? c + i : f;
-        first = first < 0 ? f : first;
+        for (int q = 0; q < 4; ++q) {
+            if (c0 + q * N >= nrp) break;
+            const int i = c0 + q * N + l;
+            const float a = (W == N || l < N) && i < nrp ? aval(u[q]) : 0.0f;
+            const float a1 = l == 0 ? carry + a : a;
+            float x = a1;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) last = aval(u[i]) > 0.0f ? c + i : last;
+            for (int k = 1; k < N; ++k) {
+                const float t = dppf<DPP_ROW_SHR1>(x) + a1;
+                x = (N == 16 || l > 0) ? t : a1;
+            }
+            const int f = a > 0.0f && w <= x ? i : NONE;
+            first = f < first ? f : first;
+            carry = W <= 16 ? gbcast_last<W>(x, l) : __shfl(x, N - 1, W);
+        }
     }
-    return sel + (first >= 0 ? first : last) * G;
+    first = gmini<N>(first);
+    if (W > 16) first = __shfl(first, 0, W);             // the other rows hold no reactions
+    if (first == NONE) {                                 // rounding left w above every sum: the last positive one
+        int last = -1;
+        for (int i = l; i < nrp; i += W) last = aval(A[sel + i * G]) > 0.0f ? i : last;
+        for (int d = W / 2; d > 0; d >>= 1) {
+            const int o = __shfl_xor(last, d, W);
+            last = o > last ? o : last;
+        }
+        first = last;
+    }
+    return sel + first * G;
 }
 
 template <int W>
@@ -1065,25 +1104,33 @@ __device__ __forceinline__ bool gssa_run(const KParams& p, GLane& L, const GView
     const uint4* SR = reinterpret_cast<const uint4*>(p.T + p.oSR);
     const uint4* DR = reinterpret_cast<const uint4*>(p.T + p.oDR);
     double tnext = L.cursor < (uint32_t)p.K ? p.ts[L.cursor] : 0.0;        // the next sample time
+    constexpr int SB = W > G || G <= 4 ? 16 : 4;
     for (int step = 0; step < n; ++step) {
         float P = 0.0f;
         const int nrp = group_rpad(p.R, G) / G;        // rounds over A with its zero padding
-        for (int r0 = 0; r0 < nrp; r0 += 4) {          // padding adds an exact 0
-            uint32_t u[4];
+        for (int r0 = 0; r0 < nrp; r0 += SB) {         // padding adds an exact 0
+            uint32_t u[SB];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) u[i] = r0 + i < nrp ? V.A[la + (r0 + i) * G] : 0u;
+            for (int q = 0; q < SB; q += 4)            // SB reads in flight
+                if (SB == 4 || r0 + q < nrp) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) P = P + aval(u[i]);
+                    for (int i = q; i < q + 4; ++i) u[i] = V.A[la + (r0 + i < nrp ? r0 + i : nrp - 1) * G];
+                }
+#pragma unroll
+            for (int q = 0; q < SB; q += 4)
+                if (SB == 4 || r0 + q < nrp) {
+#pragma unroll
+                    for (int i = q; i < q + 4; ++i) P = P + (r0 + i < nrp ? aval(u[i]) : 0.0f);
+                }
         }
         const float Pown = P;
         P = gscan<G>(P, la);
         const float a0 = gbcast_last<G>(P, la);
-        if (a0 == 0.0f) { gabsorb<W>(p, L, X, l); L.ssa_left = 0; return true; }
+        const uint64_t cand = gballot<G>(Pown > 0.0f);
+        if (a0 == 0.0f || cand == 0) { gabsorb<W>(p, L, X, l); L.ssa_left = 0; return true; }   // no lane: only with a NaN
         uint32_t w0, w1;
         grng_pair<W>(L.gg, l, w0, w1);
-        const float r1 = u32_oc(w0) * a0;
-        const int j = W < 4 ? gselect_walk<G>(p, V.A, Pown, P, r1, la) : gselect<G, W>(p, V.A, Pown, P, r1, l, 0);
-        if (j < 0) { gabsorb<W>(p, L, X, l); L.ssa_left = 0; return true; }    // unreachable for finite a0
+        const int j = gselect_ssa<G, W>(V.A, cand, Pown, P, u32_oc(w0) * a0, l, nrp);
         const uint4 sr = SR[j];              // {first change entry, count, first dependent, count}
         const float dt = u32_exp(w1) / a0;
         CTL_PHASE(PH_SSA_SELECT);
