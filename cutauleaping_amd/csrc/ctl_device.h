@@ -249,13 +249,21 @@ __device__ __forceinline__ int32_t poisson(Rng& g, float lam, const float* __res
         const float p0 = dexpf(-lam);
         for (;;) {
             const float u = rng_co(g);
+            // terms in batches of seven (63 = 9 x 7): the reciprocals are read
+            // together and one branch follows the batch; the count is the
+            // number of cumulative sums not above u
             float p = p0, F = p0;
-            int k = 0;
-            while (u >= F) {
-                ++k;
-                if (k > 63) break;
-                p = (p * lam) * recip[k];
-                F = F + p;
+            int k = u >= F ? 1 : 0;
+            for (int b = 0; k > b && b < 63; b += 7) {
+                float r[7];
+#pragma unroll
+                for (int i = 0; i < 7; ++i) r[i] = recip[b + 1 + i];
+#pragma unroll
+                for (int i = 0; i < 7; ++i) {
+                    p = (p * lam) * r[i];
+                    F = F + p;
+                    k += u >= F ? 1 : 0;
+                }
             }
             if (k <= 63) return k;
         }

@@ -939,37 +939,57 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         // these gaps), counted as a gap when it is used.
         double pos2 = pos + (double)exp_rv(L.lg);
         bool have2 = true;
+        // Rounds in batches of four: their reads are in flight together, and
+        // the events in the batch's span of the running sum are walked by one
+        // loop (one turn per event of the busiest lane) instead of a loop per
+        // reaction.
         const int nit = (p.R + G - 1) / G;
-        for (int i = 0; i < nit; ++i) {
-            const int j = la + i * G;
-            bool need = false;
-            {                                          // past R: the zero padding of A and Kc
-                const uint32_t u = V.A[j];
-                const bool crit = (u & 0x80000000u) != 0u;
-                const float lam = tau * __uint_as_float(u);
-                need = !crit && !(lam < 1.0f);
-                const bool small = !crit && lam < 1.0f && lam > 0.0f;
-                int32_t k = (crit && attempt == 0 && j == pick) ? 1 : 0;
+        for (int i0 = 0; i0 < nit; i0 += 4) {
+            uint32_t u[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) u[q] = V.A[la + (i0 + q < nit ? i0 + q : nit - 1) * G];
+            double cs[4];
+            int32_t k[4];
+            bool need[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {              // past R: the zero padding of A
+                const int j = la + (i0 + q) * G;
+                const bool in = i0 + q < nit;
+                const bool crit = (u[q] & 0x80000000u) != 0u;
+                const float lam = tau * __uint_as_float(u[q]);
+                need[q] = in && !crit && !(lam < 1.0f);
+                const bool small = in && !crit && lam < 1.0f && lam > 0.0f;
+                k[q] = (crit && attempt == 0 && j == pick) ? 1 : 0;
                 cum = small ? cum + (double)lam : cum;
-                // pos >= cum held before this reaction, so only a lane whose
-                // process mass grew draws gaps
-                while (pos < cum) {
-                    ++k;
-                    if (have2) {
-                        pos = pos2;
-                        have2 = false;
-                    } else {
-                        pos = pos + (double)exp_rv(L.lg);
+                cs[q] = cum;
+            }
+            // pos >= cum held before this batch; an event belongs to the first
+            // reaction whose running sum lies above it
+            while (pos < cum) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) k[q] += pos < cs[q] && (q == 0 || !(pos < cs[q - 1])) ? 1 : 0;
+                if (have2) {
+                    pos = pos2;
+                    have2 = false;
+                } else {
+                    pos = pos + (double)exp_rv(L.lg);
+                }
+                if (own) L.gaps++;
+            }
+            if (own) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (i0 + q < nit) {
+                        V.Kc[la + (i0 + q) * G] = k[q];      // a queued reaction's count is drawn below
+                        fk += (uint32_t)k[q];
                     }
-                    if (own) L.gaps++;
-                }
-                if (own) {
-                    V.Kc[j] = k;                     // a queued reaction's count is drawn below
-                    fk += (uint32_t)k;
-                }
             }
             // the queue's order is free: each count comes from its reaction's own stream
-            if (need && own) Q[atomicAdd(V.qn, 1u)] = (uint16_t)j;
+            if (own && (need[0] || need[1] || need[2] || need[3])) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (need[q]) Q[atomicAdd(V.qn, 1u)] = (uint16_t)(la + (i0 + q) * G);
+            }
         }
         gsync();
         CTL_PHASE(PH_COUNTS);
