@@ -844,7 +844,26 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         const uint32_t len = TC[p.oVRm + r];
         const uint32_t spw = SPI[r * W];             // species | HOR << 16 | HORtype << 24
         float mu = 0.0f, sg = 0.0f;
-        if (kuse(p.vhalf)) {
+        if (kuse(p.vhalf) == 2) {
+            // every coefficient is 0 or a power of two: v a and v (v a) are
+            // exact, so the fused additions round as the separate ones do
+            const char* Ab = reinterpret_cast<const char*>(V.A);
+            for (uint32_t k = 0; k < len; k += 4) {  // len is a multiple of 4
+                uint32_t e[4];
+                int32_t u[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) e[i] = E[(k + i) * W];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) u[i] = *reinterpret_cast<const int32_t*>(Ab + (e[i] & 0xffffu));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float v = (float)__builtin_bit_cast(_Float16, (uint16_t)(e[i] >> 16));
+                    const float a = __int_as_float(u[i] > 0 ? u[i] : 0);     // critical: 0, see below
+                    mu = fmaf(v, a, mu);
+                    sg = fmaf(v, v * a, sg);
+                }
+            }
+        } else if (kuse(p.vhalf)) {
             // entries (coefficient as FP16 << 16 | byte offset of A[reaction]):
             // both halves are read as operand selects, and v * v in FP32 is exact
             const char* Ab = reinterpret_cast<const char*>(V.A);
@@ -1013,29 +1032,60 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         CTL_PHASE(PH_POISSON);
         bool bad = false;
         const uint32_t* F = p.T + p.oFRe + l;
-        for (int r = 0; r < nrs; ++r) {
-            const uint32_t len = TC[p.oFRm + r];
-            const uint32_t sp = SPI[r * W] & 0xffffu;
-            if (sp < (uint32_t)p.S) {
-                int64_t x = X[sp];
-                bool bs = false;
-                for (uint32_t k = 0; k < len; k += 4) {   // len is a multiple of 4; padding adds 0
-                    uint32_t e[4];
-                    int32_t kc[4];
+        const char* Kb = reinterpret_cast<const char*>(V.Kc);
+        // While every lane drew fewer than flim / W firings, the counts are
+        // below 2^23 and no partial sum leaves (-2^30, 2^31 + 2^30): its bit 31
+        // says that it left [0, 2^31), and the sums fit 32 bits (a 64-bit
+        // multiply-add issues at a quarter of the rate).
+        if (__ballot(f >= (uint64_t)(p.flim / (uint32_t)W)) == 0) {
+            for (int r = 0; r < nrs; ++r) {
+                const uint32_t len = TC[p.oFRm + r];
+                const uint32_t sp = SPI[r * W] & 0xffffu;
+                if (sp < (uint32_t)p.S) {
+                    int32_t x = X[sp], any = 0;
+                    for (uint32_t k = 0; k < len; k += 4) {   // len is a multiple of 4; padding adds 0
+                        uint32_t e[4];
+                        int32_t kc[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) e[i] = F[(k + i) * W];
+                        for (int i = 0; i < 4; ++i) e[i] = F[(k + i) * W];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) kc[i] = V.Kc[e[i] & 0xffffu];
+                        for (int i = 0; i < 4; ++i) kc[i] = *reinterpret_cast<const int32_t*>(Kb + (e[i] & 0xffffu));
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        x += (int64_t)(int16_t)(e[i] >> 16) * (int64_t)kc[i];
-                        bs = bs || x < 0 || x > 2147483647LL;
+                        for (int i = 0; i < 4; ++i) {
+                            x = __mul24((int)(int16_t)(e[i] >> 16), kc[i]) + x;
+                            any |= x;
+                        }
                     }
+                    X1[sp] = x;
+                    bad = bad || any < 0;
                 }
-                X1[sp] = (int32_t)x;
-                bad = bad || bs;
+                F += len * W;
             }
-            F += len * W;
+        } else {
+            for (int r = 0; r < nrs; ++r) {
+                const uint32_t len = TC[p.oFRm + r];
+                const uint32_t sp = SPI[r * W] & 0xffffu;
+                if (sp < (uint32_t)p.S) {
+                    int64_t x = X[sp];
+                    bool bs = false;
+                    for (uint32_t k = 0; k < len; k += 4) {
+                        uint32_t e[4];
+                        int32_t kc[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) e[i] = F[(k + i) * W];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) kc[i] = *reinterpret_cast<const int32_t*>(Kb + (e[i] & 0xffffu));
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            x += (int64_t)(int16_t)(e[i] >> 16) * (int64_t)kc[i];
+                            bs = bs || x < 0 || x > 2147483647LL;
+                        }
+                    }
+                    X1[sp] = (int32_t)x;
+                    bad = bad || bs;
+                }
+                F += len * W;
+            }
         }
         fired = gsum64<W>(f);
         const bool any_bad = gballot<W>(bad) != 0;
@@ -1675,10 +1725,11 @@ inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, in
     // var entries: with every |coefficient| <= 2048 (exact in FP16, v * v exact
     // in FP32) and A's byte offsets below 2^16, as FP16 coefficient << 16 |
     // byte offset of A[reaction]; else reaction | v << 16
-    p.vhalf = 4 * (m.R + 1) <= 0xffff ? 1 : 0;
+    p.vhalf = 4 * (m.R + 1) <= 0xffff ? 2 : 0;
     for (uint32_t e : m.Vent) {
         const int v = (int)(int16_t)(e >> 16);
         if (v > 2048 || v < -2048) p.vhalf = 0;
+        else if ((v & -v) != v && ((-v) & v) != -v && p.vhalf) p.vhalf = 1;
     }
     if (p.vhalf) {
         std::vector<uint32_t> vent(m.Vent.size());
@@ -1690,7 +1741,17 @@ inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, in
     } else {
         rounds(W, sorder, m.Vptr, m.Vent, p.oVRm, p.oVRe, 4, 0, (uint32_t)m.R);       // padding: the zero slot A[R]
     }
-    rounds(W, sorder, FSptr, FSent, p.oFRm, p.oFRe, 4, 0, 0u);
+    // change entries as byte offset of Kc[reaction] (R <= 8191: a group's LDS
+    // holds 16384 words) | change << 16; flim: firings of a leap below which
+    // the update's sums fit 32 bits
+    std::vector<uint32_t> fent(FSent.size());
+    int vmax = 1;
+    for (size_t h = 0; h < FSent.size(); ++h) {
+        vmax = std::max(vmax, std::abs((int)(int16_t)(FSent[h] >> 16)));
+        fent[h] = (FSent[h] & 0xffff0000u) | (FSent[h] & 0xffffu) * 4u;
+    }
+    p.flim = std::min(1u << 23, (1u << 30) / (uint32_t)vmax);
+    rounds(W, sorder, FSptr, fent, p.oFRm, p.oFRe, 4, 0, 0u);
 }
 
 }  // namespace ctl

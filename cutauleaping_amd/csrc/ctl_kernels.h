@@ -74,13 +74,15 @@ struct KParams {
     // var and fear round lengths are multiples of 4 (loads issue 4 at a time).
     // Reactant entries (species | multiplicity << 16; with pfast the index of
     // the reactant's factor in the group's factor table, padding 2S), var
-    // entries of the tau' sums and species-major fear entries (reaction |
-    // change << 16).
+    // entries of the tau' sums and species-major fear entries (byte offset of
+    // the reaction's count | change << 16).
     // Var and fear rounds list species in the order T[oSPI + r*G + l]
     // (species | HOR << 16 | HORtype << 24; 0xffffffff: none), longest lists
     // first.  gsimple: no species has HOR 3 or HOR 2 of type 2, so g is 1 or 2.
     int oPRm, oPRe, oVRm, oVRe, oFRm, oFRe, oSPI, gsimple;
-    int vhalf;                // var entries as FP16 coefficient << 16 | byte offset of A[reaction] (every |v| <= 2048)
+    int vhalf;                // var entries as FP16 coefficient << 16 | byte offset of A[reaction] (every |v| <= 2048);
+                              //   2: every coefficient is a power of two
+    uint32_t flim;            // leap firings below which the update's 32-bit sums are exact
     int oSR;                  // per reaction {first change entry (word of T), count, first dependent, count} (uint4)
     int oDR;                  // pfast 1 / 2: SSA dependent records {r, entry 0, entry 1, rate} (uint4, Dptr order),
                               //   the entries as factor indices (1) or species | multiplicity << 16 (2)
