@@ -299,6 +299,23 @@ __device__ __forceinline__ uint64_t gsum64(uint64_t v) {
     return v;
 }
 
+// Sum of uint32 over the group (the caller knows that it fits).
+template <int G>
+__device__ __forceinline__ uint32_t gsum32(uint32_t v) {
+    auto step = [&](int o) { v += (uint32_t)o; };
+    if (G >= 2) step(__builtin_amdgcn_update_dpp(0, (int)v, DPP_QP_1032, 0xf, 0xf, false));
+    if (G >= 4) step(__builtin_amdgcn_update_dpp(0, (int)v, DPP_QP_2301, 0xf, 0xf, false));
+    if (G >= 8) step(__builtin_amdgcn_update_dpp(0, (int)v, DPP_ROW_HALF_MIRROR, 0xf, 0xf, false));
+    if (G >= 16) step(__builtin_amdgcn_update_dpp(0, (int)v, DPP_ROW_MIRROR, 0xf, 0xf, false));
+    if (G >= 32) {                                  // add the rows' sums
+        const uint32_t r0 = __builtin_amdgcn_readlane(v, 15), r1 = __builtin_amdgcn_readlane(v, 31);
+        const uint32_t r2 = __builtin_amdgcn_readlane(v, 47), r3 = __builtin_amdgcn_readlane(v, 63);
+        if (G == 64) v = (r0 + r1) + (r2 + r3);
+        else v = (threadIdx.x & 32u) ? r2 + r3 : r0 + r1;
+    }
+    return v;
+}
+
 // Group state: the scalars are identical in every lane of the group; the
 // Poisson / gap counters are per lane and summed when the simulation ends.
 // The group's stream (counter word 3 = 0) with its Philox blocks spread over
@@ -539,15 +556,25 @@ __device__ __forceinline__ void gprops_wide(const KParams& p, const int32_t* X, 
     P = 0.0f;
     PC = 0.0f;
     const int nrp = group_rpad(p.R, G) / G;
-    for (int r0 = 0; r0 < nrp; r0 += 4) {              // padding adds an exact 0
-        uint32_t u[4];
+    constexpr int D = W > 16 ? 16 : 4;                 // reads in flight
+    for (int r0 = 0; r0 < nrp; r0 += D) {
+        uint32_t u[D];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) u[i] = r0 + i < nrp ? A[a0 + (r0 + i) * G] : 0u;
+        for (int q = 0; q < D; q += 4)
+            if (r0 + q < nrp) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            P = P + aval(u[i]);
-            if (u[i] & 0x80000000u) PC = PC + aval(u[i]);
-        }
+                for (int i = q; i < q + 4; ++i) u[i] = A[a0 + (r0 + i < nrp ? r0 + i : nrp - 1) * G];
+            }
+#pragma unroll
+        for (int q = 0; q < D; q += 4)
+            if (r0 + q < nrp) {
+#pragma unroll
+                for (int i = q; i < q + 4; ++i) {
+                    const float a = r0 + i < nrp ? aval(u[i]) : 0.0f;
+                    P = P + a;
+                    PC = PC + ((u[i] & 0x80000000u) ? a : 0.0f);
+                }
+            }
     }
 }
 
@@ -812,6 +839,19 @@ __device__ __forceinline__ void gabsorb(const KParams& p, GLane& L, const int32_
     L.absorbed = 1;
 }
 
+// Four entries of a lane's round list from entry k on, one batch ahead of
+// their use: without the barrier the compiler moves the loads back there.
+// Taken by teams of more than 16 lanes, which wait for the L1 / L2 and not
+// for issue slots: 200 reactions, 1000 simulations at W = 64 67.9 -> 66.9 ms,
+// 300 reactions at G = W = 64 66.8 -> 64.7 ms; at W = 16, full chip, the four
+// more registers cost 79.1 -> 82.3 ms.
+template <int W>
+__device__ __forceinline__ void gentries(const uint32_t* E, uint32_t k, uint32_t (&e)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) e[i] = E[(k + i) * W];
+    asm volatile("" ::: "memory");
+}
+
 // One adaptive leap attempt (PreCalculations, T.cu:1568-2093).
 template <int G, int W, int PFM = 3>
 __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V, int l,
@@ -819,6 +859,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
     if (L.t >= p.tmax) return LEAP_DONE;
     const int la = l & (G - 1);              // the algorithm's lane this one stands for
     const bool own = l < G;                  // one lane per algorithm lane counts
+    constexpr bool kAhead = W > 16 && (W > G || W == 64);    // see gentries
     int32_t* X = V.Xb + (L.xb ? p.S : 0);
     int32_t* X1 = V.Xb + (L.xb ? 0 : p.S);
     float P, PC;
@@ -848,11 +889,19 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
             // every coefficient is 0 or a power of two: v a and v (v a) are
             // exact, so the fused additions round as the separate ones do
             const char* Ab = reinterpret_cast<const char*>(V.A);
+            uint32_t en[4];
+            if (kAhead && len > 0) gentries<W>(E, 0u, en);
             for (uint32_t k = 0; k < len; k += 4) {  // len is a multiple of 4
                 uint32_t e[4];
                 int32_t u[4];
+                if (kAhead) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) e[i] = E[(k + i) * W];
+                    for (int i = 0; i < 4; ++i) e[i] = en[i];
+                    gentries<W>(E, k + 4 < len ? k + 4 : k, en);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) e[i] = E[(k + i) * W];
+                }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) u[i] = *reinterpret_cast<const int32_t*>(Ab + (e[i] & 0xffffu));
 #pragma unroll
@@ -867,11 +916,19 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
             // entries (coefficient as FP16 << 16 | byte offset of A[reaction]):
             // both halves are read as operand selects, and v * v in FP32 is exact
             const char* Ab = reinterpret_cast<const char*>(V.A);
+            uint32_t en[4];
+            if (kAhead && len > 0) gentries<W>(E, 0u, en);
             for (uint32_t k = 0; k < len; k += 4) {  // len is a multiple of 4
                 uint32_t e[4];
                 int32_t u[4];
+                if (kAhead) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) e[i] = E[(k + i) * W];
+                    for (int i = 0; i < 4; ++i) e[i] = en[i];
+                    gentries<W>(E, k + 4 < len ? k + 4 : k, en);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) e[i] = E[(k + i) * W];
+                }
 #pragma unroll
                 for (int i = 0; i < 4; ++i) u[i] = *reinterpret_cast<const int32_t*>(Ab + (e[i] & 0xffffu));
 #pragma unroll
@@ -1043,11 +1100,19 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
                 const uint32_t sp = SPI[r * W] & 0xffffu;
                 if (sp < (uint32_t)p.S) {
                     int32_t x = X[sp], any = 0;
+                    uint32_t en[4];
+                    if (kAhead && len > 0) gentries<W>(F, 0u, en);
                     for (uint32_t k = 0; k < len; k += 4) {   // len is a multiple of 4; padding adds 0
                         uint32_t e[4];
                         int32_t kc[4];
+                        if (kAhead) {
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) e[i] = F[(k + i) * W];
+                            for (int i = 0; i < 4; ++i) e[i] = en[i];
+                            gentries<W>(F, k + 4 < len ? k + 4 : k, en);
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) e[i] = F[(k + i) * W];
+                        }
 #pragma unroll
                         for (int i = 0; i < 4; ++i) kc[i] = *reinterpret_cast<const int32_t*>(Kb + (e[i] & 0xffffu));
 #pragma unroll
@@ -1061,7 +1126,9 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
                 }
                 F += len * W;
             }
+            if (W > 16) fired = gsum32<W>((uint32_t)f);
         } else {
+            if (W > 16) fired = gsum64<W>(f);
             for (int r = 0; r < nrs; ++r) {
                 const uint32_t len = TC[p.oFRm + r];
                 const uint32_t sp = SPI[r * W] & 0xffffu;
@@ -1087,7 +1154,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
                 F += len * W;
             }
         }
-        fired = gsum64<W>(f);
+        if (W <= 16) fired = gsum64<W>(f);
         const bool any_bad = gballot<W>(bad) != 0;
         gsync();
         CTL_PHASE(PH_UPDATE);
