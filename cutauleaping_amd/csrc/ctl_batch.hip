@@ -38,6 +38,7 @@
 #include "ctl_gbatch.h"
 #include "ctl_group.h"
 #include "ctl_kernels.h"
+#include "ctl_stat.h"
 
 #pragma clang fp contract(off)
 
@@ -147,6 +148,12 @@ __global__ __launch_bounds__(256) void batch_kernel(BatchParams bp) {
     if (L.sim >= 0) store_lane(desc_of(bp, m), L);
 }
 
+// Statistics of all models: one workgroup per model.
+__global__ __launch_bounds__(STAT_BLOCK) void batch_stat_kernel(const KParams* __restrict__ desc,
+                                                                unsigned long long* tot) {
+    const KParams& p = desc[blockIdx.x];
+    stat_add(p.simstat, threadIdx.x, p.n, STAT_BLOCK, tot);
+}
 
 }  // namespace ctl
 
@@ -185,6 +192,7 @@ struct ctl_batch {
     std::vector<int> K, SS, lanes;
     KParams* d_desc = nullptr;
     uint32_t* d_rep_next = nullptr;            // per-model replica counters
+    unsigned long long* d_tot = nullptr;       // batch_stat_kernel's totals
     uint32_t* h_done = nullptr;                // per-class done counters (pinned host memory)
     std::vector<BClass> classes;
     int verbose = 0;
@@ -407,7 +415,7 @@ int ctl_batch_create_lanes(const ctl_model* const* models, const int64_t* replic
             if (lanes[i] == G) { c.models.push_back(i); c.total += replicas[i]; }
         if (!c.models.empty()) b->classes.push_back(c);
     }
-    if ((rc = balloc(b, &b->d_rep_next, nmodels))) return bail(rc);
+    if ((rc = balloc(b, &b->d_rep_next, nmodels)) || (rc = balloc(b, &b->d_tot, ST_COUNT))) return bail(rc);
     if ((e = hipHostMalloc((void**)&b->h_done, sizeof(uint32_t) * b->classes.size(), hipHostMallocDefault)) != hipSuccess)
         return bail(bhip(e, "hipHostMalloc"));
     std::vector<int> cls(nmodels, -1);
@@ -639,6 +647,7 @@ int ctl_batch_run(ctl_batch* b) {
     }
     // replica counters of every model (before any class starts)
     BHIP(hipMemset(b->d_rep_next, 0, sizeof(uint32_t) * b->nmodels), "memset");
+    BHIP(hipMemset(b->d_tot, 0, ST_COUNT * sizeof(*b->d_tot)), "memset");
     ctl_stats& S = b->stats;
     S.launches = 0;
     // The classes run concurrently: each round launches every unfinished
@@ -687,15 +696,13 @@ int ctl_batch_run(ctl_batch* b) {
         if (S.launches >= (1 << 20)) return ctl::fail(CTL_E_STATE, "batch did not finish");
     }
     S.kernel_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - k0).count();
-    S.firings = S.leaps = S.rejections = S.switches = S.ssa_steps = S.poisson = S.gaps = S.absorbed = 0;
-    for (int i = 0; i < b->nmodels; ++i) {
-        std::vector<ctl_sim_stat> st(b->desc[i].n);
-        BHIP(hipMemcpy(st.data(), b->desc[i].simstat, sizeof(ctl_sim_stat) * st.size(), hipMemcpyDeviceToHost), "D2H");
-        for (const auto& x : st) {
-            S.firings += x.firings; S.leaps += x.leaps; S.rejections += x.rejections; S.switches += x.switches;
-            S.ssa_steps += x.ssa_steps; S.poisson += x.poisson; S.gaps += x.gaps; S.absorbed += x.absorbed;
-        }
-    }
+    unsigned long long tot[ST_COUNT];
+    hipStream_t st0 = b->classes[0].stream;
+    hipLaunchKernelGGL(batch_stat_kernel, dim3(b->nmodels), dim3(STAT_BLOCK), 0, st0, b->d_desc, b->d_tot);
+    BHIP(hipGetLastError(), "batch_stat_kernel launch");
+    BHIP(hipMemcpyAsync(tot, b->d_tot, sizeof tot, hipMemcpyDeviceToHost, st0), "hipMemcpy D2H");
+    BHIP(hipStreamSynchronize(st0), "hipStreamSynchronize");
+    stat_store(S, tot);
     S.simulations = (uint64_t)b->total;
     S.wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
     b->ran = true;

@@ -31,6 +31,7 @@
 #include "ctl_internal.h"
 #include "ctl_kernels.h"
 #include "ctl_small.h"
+#include "ctl_stat.h"
 
 #pragma clang fp contract(off)
 
@@ -190,6 +191,13 @@ const void* group_kernel_fn(int G, int W, bool rg, int pf) {
     return nullptr;
 }
 
+// Statistics of all simulations; at most 128 workgroups, so that the atomics
+// on the eight totals stay few.
+__global__ __launch_bounds__(STAT_BLOCK) void stat_kernel(const ctl_sim_stat* __restrict__ st, int n,
+                                                          unsigned long long* tot) {
+    stat_add(st, blockIdx.x * STAT_BLOCK + threadIdx.x, n, gridDim.x * STAT_BLOCK, tot);
+}
+
 // Reference sample layout [i][sk][sim] from the kernel's [sim][i][sk].
 __global__ void to_reference_layout(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, int n, int KS) {
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -332,6 +340,7 @@ struct ctl_sim {
     std::vector<void*> allocs;
     bool ran = false;
     ctl_stats stats{};
+    unsigned long long* d_tot = nullptr;     // stat_kernel's totals
     // fitness
     uint32_t* d_target = nullptr;
     int8_t* d_t2e = nullptr;
@@ -801,7 +810,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
     }
     if ((rc = dalloc(s, &p.storage, (size_t)n * K * SS)) || (rc = dalloc(s, &p.simstat, n)) ||
         (rc = dalloc(s, &p.xfinal, (size_t)n * S)) || (rc = dalloc(s, &p.tfinal, n)) ||
-        (rc = dalloc(s, &p.next_sim, 2)))
+        (rc = dalloc(s, &p.next_sim, 2)) || (rc = dalloc(s, &s->d_tot, ST_COUNT)))
         return bail(rc);
     p.done = p.next_sim + 1;
     s->stats.slots = ns;
@@ -822,6 +831,7 @@ int ctl_sim_run(ctl_sim* s) {
     HIPCHK(hipMemsetAsync(p.storage, 0, sizeof(uint32_t) * (size_t)s->n * p.K * p.SS, s->stream), "memset");
     HIPCHK(hipMemsetAsync(s->sst.sim, 0xff, sizeof(int32_t) * s->ns, s->stream), "memset");
     HIPCHK(hipMemsetAsync(p.next_sim, 0, 2 * sizeof(uint32_t), s->stream), "memset");
+    HIPCHK(hipMemsetAsync(s->d_tot, 0, ST_COUNT * sizeof(*s->d_tot), s->stream), "memset");
     ctl_stats& S = s->stats;
     S.kernel_ms = 0.0;
     S.launches = 0;
@@ -863,14 +873,13 @@ int ctl_sim_run(ctl_sim* s) {
     }
     S.kernel_ms = total_ms;
     // totals
-    std::vector<ctl_sim_stat> st(s->n);
-    HIPCHK(hipMemcpy(st.data(), p.simstat, sizeof(ctl_sim_stat) * s->n, hipMemcpyDeviceToHost), "hipMemcpy D2H");
-    S.firings = S.leaps = S.rejections = S.switches = S.ssa_steps = S.poisson = S.gaps = S.absorbed = 0;
-    for (const auto& x : st) {
-        S.firings += x.firings; S.leaps += x.leaps; S.rejections += x.rejections; S.switches += x.switches;
-        S.ssa_steps += x.ssa_steps; S.poisson += x.poisson; S.gaps += x.gaps;
-        S.absorbed += x.absorbed;
-    }
+    unsigned long long tot[ST_COUNT];
+    const int sblocks = std::min((s->n + STAT_BLOCK - 1) / STAT_BLOCK, 128);
+    hipLaunchKernelGGL(stat_kernel, dim3(sblocks), dim3(STAT_BLOCK), 0, s->stream, p.simstat, s->n, s->d_tot);
+    HIPCHK(hipGetLastError(), "stat_kernel launch");
+    HIPCHK(hipMemcpyAsync(tot, s->d_tot, sizeof tot, hipMemcpyDeviceToHost, s->stream), "hipMemcpy D2H");
+    HIPCHK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
+    stat_store(S, tot);
     S.simulations = (uint64_t)s->n;
     S.wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - w0).count();
     s->ran = true;
