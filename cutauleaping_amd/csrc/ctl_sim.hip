@@ -593,14 +593,17 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
     if (G > 1) {
         const size_t gwords = group_lds_words(S, R, G);    // group LDS words per simulation
         if (gwords * 4 > 65536) return bail(ctl::fail(CTL_E_LIMIT, "model too large for the group kernel (more than 64 KB of LDS)"));
-        // regrouping simulations by mode (leap / SSA) every `compact` iterations;
-        // by default for groups of 16 or more lanes (networks of more than 128
-        // reactions, where a leap costs several SSA steps) and never in
-        // force-SSA mode, where every simulation is in one mode (measured: the
-        // 100x200 network, G = 16: +10 %; the 50x100 sweep network, G = 8:
-        // -6 %; the SSA-dominated enzyme cascade, G = 4: -40 %)
-        const int compact = o->compact_interval > 0 ? o->compact_interval
-                            : (o->compact_interval < 0 || o->force_ssa || G < 16) ? 0 : 8;
+        // Regrouping simulations by mode (leap / SSA) every `compact` iterations
+        // is done on request only: a wavefront whose groups are in both modes
+        // loses less than the barrier, the second wavefront of the workgroup
+        // and the hand-over of registers cost (groups already gather their
+        // bursts, GBURST_WAIT).  Kernel times in ms, off / every 8:
+        //   100x200 network, G = 16, n = 12000, t = 2   200 / 226
+        //                            n = 16384, t = 2   228 / 230, t = 50: 1246 / 1249
+        //                            n = 65536, t = 2   815 / 902
+        //   80x300 network, G = 32, n = 16384, t = 0.5  684 / 723
+        //   50x100 sweep network, G = 8, n = 32768      402 / 459
+        const int compact = o->compact_interval > 0 ? o->compact_interval : 0;
         // groups per workgroup: block_size / G when given (64..256), else two
         // wavefronts when regrouping (fewer wavefronts wait for the slowest at
         // each regrouping: C1 +1.5 % over four) and four otherwise

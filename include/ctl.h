@@ -89,9 +89,8 @@ typedef struct {
     int32_t  compact_interval; /* every this many iterations a workgroup of several wavefronts
                                   regroups its simulations so that leap-mode and SSA-mode ones run
                                   in different wavefronts, SSA bursts then running ssa_chunk steps
-                                  per iteration; trajectories do not depend on it.  0: library
-                                  default (8 for 16 or 32 lanes per simulation outside
-                                  force-SSA mode, else never), < 0: never */
+                                  per iteration; trajectories do not depend on it.  0 (the
+                                  library's default) and < 0: never */
 } ctl_opts;
 
 typedef struct {
