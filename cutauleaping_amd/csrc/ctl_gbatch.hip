@@ -130,9 +130,8 @@ __global__ __launch_bounds__(64) void gbatch_kernel(GBatchParams bp) {
 }
 
 // Group batch, G = 2..32 (see GClassParams).  The loop mirrors group_kernel:
-// one leap attempt per group per iteration, SSA bursts held until a second
-// group of the wavefront switches (at most GBURST_WAIT iterations, or until
-// every group with a replica waits); a group without a replica idles.  Each
+// one leap attempt per group per iteration, SSA bursts held until one
+// group has waited GBURST_WAIT iterations or every group with a replica waits; a group without a replica idles.  Each
 // replica's trajectory depends only on its own state and streams.
 template <int G, int W>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(gwaves(G, W))))
@@ -222,7 +221,7 @@ void gclass_kernel(GClassParams bp) {
         }
         const uint64_t lead = __ballot(l == 0 && active);       // groups holding a replica
         const uint64_t pm = __ballot(pend && l == 0);           // ... waiting for a burst
-        const bool go = pm != 0 && (__popcll(pm) >= 2 || pm == lead || __ballot(pend && waited >= GBURST_WAIT) != 0);
+        const bool go = pm != 0 && (pm == lead || __ballot(pend && waited >= GBURST_WAIT) != 0);
         if (go && pend) {
             pend = false;
             if (gssa<G, W>(p, L, V, l)) gfinish<W>(p, L, V, l);

@@ -1408,8 +1408,17 @@ __device__ __forceinline__ void gfinish(const KParams& p, GLane& L, const GView&
     L.sim = -1;
 }
 
-// Longest a switched group waits for a partner burst (leap iterations).
-constexpr int GBURST_WAIT = 24;
+// Longest a switched group waits for the bursts of the wavefront's other
+// groups (leap iterations).  A burst of 100 steps idles every group that is
+// not in one, so they gather: when one has waited this long, or all have
+// switched, all that have switched run theirs.  Going as soon as two had
+// switched cost more the more groups share the wavefront.  Kernel times in ms,
+// two or 24 / all or 4 / 6 / 10 / 16 / 28:
+//   100x200 network, 4 groups, t = 50      1250 / 1206 / 1184 / 1161 / 1176 / 1247
+//   50x100 network, 8 groups, t = 0.2       417 /  284 /  268 /  258 /  267 /  288
+//   50x100 sweep network, 8 groups          408 /  325 /  320 /  318 /  316 /  318
+//   20-stage cascade, 16 groups            20.2 / 18.5 / 18.4 / 18.5 / 18.5 / 18.5
+constexpr int GBURST_WAIT = 10;
 
 // ---------------------------------------------------------------------------
 // Regrouping groups by mode.  The groups of a wavefront run in lockstep: while
@@ -1526,10 +1535,9 @@ __host__ __device__ constexpr int gwaves(int G, int W) {
 // simulations from the queue; a launch runs up to p.iters iterations per
 // group (a leap attempt, or SSA steps), then parks the group's state in the
 // slot arrays for the next launch.  Without regrouping (RG false: W = 64, or
-// p.compact = 0) a group that switched to SSA holds its whole burst until a second
-// group of the wavefront switches too (or it has waited GBURST_WAIT
-// iterations, or every group still running is waiting), so that bursts run
-// side by side.  Either way each simulation's events and draws are its own;
+// p.compact = 0) a group that switched to SSA holds its whole burst until one
+// has waited GBURST_WAIT iterations or every group of the wavefront still
+// running has switched, so that bursts run side by side.  Either way each simulation's events and draws are its own;
 // only the order in which the lanes serve the simulations moves.
 template <int G, int W, bool RG, int PF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gwaves(G, W)))) void group_kernel(KParams p) {
@@ -1654,7 +1662,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gwaves(G, W
         if (W < 64) {
             const uint64_t lead = __ballot(l == 0);            // groups still in the loop
             const uint64_t pm = __ballot(pend && l == 0);       // ... waiting for a burst
-            go = pm != 0 && (__popcll(pm) >= 2 || pm == lead || __ballot(pend && waited >= GBURST_WAIT) != 0);
+            go = pm != 0 && (pm == lead || __ballot(pend && waited >= GBURST_WAIT) != 0);
         }
         if (go && pend) {
             pend = false;
