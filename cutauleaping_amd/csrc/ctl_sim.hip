@@ -617,18 +617,24 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         // Lanes that execute a simulation.  When the simulations leave lanes
         // of the chip empty, each takes W > G of them: the widest W at which
         // all n are still resident at once (one more round of simulations
-        // costs more than the wider work gains).  Kernel times in ms, W = G /
-        // 16 / 32 / 64 (resident simulations at 16, 32, 64: 16384, 8192, 3072):
-        //   100x200 network, G = 16, t = 0.5   n =   24: - / 140 / 104 / 74
-        //                                      n = 4096: - / 156 / 118 / 152
-        //                                      n = 16384: - / 201 / 304 / -
-        //   50x100 network, G = 8, t = 0.2     n =  512: 188 / 125 / 80 / 67
-        //                                      n = 8192: 204 / 141 / 112 / 211
-        //                                      n = 32768: 248 / 358 / 413 / 756
-        //   enzyme cascade, G = 4, t = 50      n = 5003: 6.2 / 5.4 / 5.2 / 5.3
+        // costs more than the wider work gains) and, below 64, leave a quarter
+        // of the places empty: with all of them taken the wavefronts compete
+        // for issue slots and the narrower team does less redundant work.
+        // Kernel times in ms, W = G / 16 / 32 / 64 (resident simulations at
+        // 16, 32: 16384, 8192):
+        //   100x200 network, G = 16, t = 0.5   n =   24: - / 121 / 93 / 65
+        //                                      n = 1000: - / 123 / 95 / 67
+        //                                      n = 4096: - / 124 / 106 / 144
+        //                                      n = 8192: - / 133 / 140 / 286
+        //   50x100 network, G = 8, t = 0.2     n =  512: 94 / 74 / 63 / 48
+        //                                      n = 6000: 96 / 82 / 80 / 153
+        //                                      n = 8192: 96 / 82 / 91 / 205
+        //                                      n = 16384: 101 / 107 / 183 / 401
+        //   enzyme cascade, G = 4, t = 50      n = 5003: 4.8 / 4.2 / 4.7 / 9.4
+        //                                      n = 16000: 4.8 / 5.4 / 10.4 / 27
         // At most 16 in force-SSA mode: an SSA step is one chain of selection
         // and update that a wider team does not shorten (cascade of 13 stages,
-        // n = 5003, force-SSA: 4.8 / 4.6 / 5.0 / 5.1).  An explicit geometry
+        // force-SSA: n = 5003 4.7 / 4.1 / 4.5 / 9.3).  An explicit geometry
         // (block_size, slots, a regrouping interval) keeps W = G.
         int W = G;
         if (o->slots <= 0 && o->block_size <= 0 && o->compact_interval <= 0)
@@ -636,7 +642,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
                 const size_t sm = (size_t)(64 / w) * gwords * 4;
                 int cu = 0;
                 e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&cu, group_kernel_fn(G, w, false, 1), 64, sm);
-                if (e == hipSuccess && (long long)prop.multiProcessorCount * cu * (64 / w) >= n) {
+                if (e == hipSuccess && (long long)prop.multiProcessorCount * cu * (64 / w) >= (w < 64 ? n + (long long)n / 3 : n)) {
                     W = w;
                     gpb = 64 / w;                             // one wavefront per workgroup
                     break;
