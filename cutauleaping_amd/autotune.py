@@ -254,7 +254,7 @@ def tune(left, right, x0, c, ts, *, feed=None, cs=None, gpu=0, probe_sims=65536,
                 if r > best_rate:
                     best, best_rate = o, r
             if 1 < G < 64 and best.get("compact_interval", 0) >= 0:
-                o = dict(best, block_size=128)      # regrouping over two wavefronts instead of four
+                o = dict(best, block_size=128)      # two wavefronts a workgroup
                 r = score(o)
                 if r > best_rate:
                     best, best_rate = o, r
@@ -275,8 +275,7 @@ def tune(left, right, x0, c, ts, *, feed=None, cs=None, gpu=0, probe_sims=65536,
             # regrouping, and the defaults at every other G that came within
             # 25 % in stage 1.
             def regroups(o):
-                ci = o.get("compact_interval", 0)
-                return ci > 0 or (ci == 0 and 16 <= o["lanes_per_sim"] < 64 and not force_ssa)
+                return o.get("compact_interval", 0) > 0
             rivals = [best] + ([{"lanes_per_sim": G}] if best != {"lanes_per_sim": G} else [])
             if 1 < G < 64:
                 other = None
