@@ -130,9 +130,10 @@ __global__ __launch_bounds__(64) void gbatch_kernel(GBatchParams bp) {
 }
 
 // Group batch, G = 2..32 (see GClassParams).  The loop mirrors group_kernel:
-// one leap attempt per group per iteration, SSA bursts held until one
-// group has waited GBURST_WAIT iterations or every group with a replica waits; a group without a replica idles.  Each
-// replica's trajectory depends only on its own state and streams.
+// one leap attempt per group per iteration, SSA bursts held until one group
+// has waited GBURST_WAIT iterations or every group with a replica waits; a
+// group without a replica idles.  Each replica's trajectory depends only on
+// its own state and streams.
 template <int G, int W>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(gwaves(G, W))))
 void gclass_kernel(GClassParams bp) {

@@ -698,15 +698,14 @@ __device__ __forceinline__ void gprops(const KParams& p, const int32_t* X, const
 // Selection: among the lanes with a positive own partial (Pown), the first
 // whose inclusive sum P reaches w, else the last such lane; then the walk
 // through that lane's reactions from the previous lane's inclusive sum
-// (which = 0: all reactions; which = 2: the critical ones plus reaction 0,
-// the reference's pick walk that starts from a_0, T.cu:1993-2006).  Lanes
+// (the critical ones plus reaction 0: the reference's pick walk starts from
+// a_0, T.cu:1993-2006).  Lanes
 // with a zero partial are skipped: the scan associates differently per lane,
 // so such a lane's inclusive sum can round above its predecessor's.  Only a
 // reaction with a positive propensity is chosen.  Returns the chosen
 // reaction (group-uniform) or -1 when no lane has a positive partial.
 template <int G, int W>
-__device__ __forceinline__ int gselect(const KParams& p, const uint32_t* A, float Pown, float P, float w, int l,
-                                       int which) {
+__device__ __forceinline__ int gselect(const KParams& p, const uint32_t* A, float Pown, float P, float w, int l) {
     const uint64_t cand = gballot<G>(Pown > 0.0f);
     if (cand == 0) return -1;
     const uint64_t hit = gballot<G>(Pown > 0.0f && P >= w);
@@ -729,7 +728,7 @@ __device__ __forceinline__ int gselect(const KParams& p, const uint32_t* A, floa
         const bool in = l < N && i < nj;
         const int j = sel + i * G;
         const uint32_t u = in ? A[j] : 0u;
-        const bool use = which != 2 || (u & 0x80000000u) || j == 0;
+        const bool use = (u & 0x80000000u) || j == 0;
         const float a = use ? aval(u) : 0.0f;
         const float a1 = l == 0 ? carry + a : a;
         float x = a1;
@@ -758,7 +757,7 @@ __device__ __forceinline__ int gmini(int v) {
     return v;
 }
 
-// gselect over all reactions (which = 0) for the SSA step, without branches
+// The same over all reactions for the SSA step, without branches
 // that depend on the simulation: a taken branch costs about 20 ns, and
 // straight-line code lets the step's exponential run between the row shifts.
 // cand: the lanes with a positive partial (not 0).  Teams narrower than 16
@@ -991,7 +990,7 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         }
         const float Qown = Q;
         Q = gscan<G>(Q, la);
-        pick = gselect<G, W>(p, V.A, Qown, Q, w, l, 2);
+        pick = gselect<G, W>(p, V.A, Qown, Q, w, l);
     }
     CTL_PHASE(PH_PICK);
     uint64_t fired = 0;
