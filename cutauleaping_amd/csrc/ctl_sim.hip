@@ -619,7 +619,10 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         // all n are still resident at once (one more round of simulations
         // costs more than the wider work gains) and, below 64, leave a quarter
         // of the places empty: with all of them taken the wavefronts compete
-        // for issue slots and the narrower team does less redundant work.
+        // for issue slots and the narrower team does less redundant work
+        // (with more than 14 reactions per algorithm lane the wider team's
+        // shorter rounds still win: 100x200 network at G = 8, n = 16384,
+        // t = 0.2, W = 8 / 16 145 / 134; 64x128 network, t = 0.5 80.5 / 79.5).
         // Kernel times in ms, W = G / 16 / 32 / 64 (resident simulations at
         // 16, 32: 16384, 8192):
         //   100x200 network, G = 16, t = 0.5   n =   24: - / 121 / 93 / 65
@@ -642,7 +645,8 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
                 const size_t sm = (size_t)(64 / w) * gwords * 4;
                 int cu = 0;
                 e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&cu, group_kernel_fn(G, w, false, 1), 64, sm);
-                if (e == hipSuccess && (long long)prop.multiProcessorCount * cu * (64 / w) >= (w < 64 ? n + (long long)n / 3 : n)) {
+                const long long need = w < 64 && R <= 14 * G ? n + (long long)n / 3 : n;
+                if (e == hipSuccess && (long long)prop.multiProcessorCount * cu * (64 / w) >= need) {
                     W = w;
                     gpb = 64 / w;                             // one wavefront per workgroup
                     break;
