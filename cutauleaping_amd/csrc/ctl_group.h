@@ -1090,15 +1090,16 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         const uint32_t* F = p.T + p.oFRe + l;
         const char* Kb = reinterpret_cast<const char*>(V.Kc);
         // While every lane drew fewer than flim / W firings, the counts are
-        // below 2^23 and no partial sum leaves (-2^30, 2^31 + 2^30): its bit 31
-        // says that it left [0, 2^31), and the sums fit 32 bits (a 64-bit
-        // multiply-add issues at a quarter of the rate).
+        // below 2^23 and no partial sum leaves (-2^30, 2^31 + 2^30): bit 31 of
+        // the sum modulo 2^32 says that it left [0, 2^31) (a 64-bit
+        // multiply-add issues at a quarter of the rate).  The sums are
+        // unsigned: a signed one beyond 2^31 - 1 has no defined value.
         if (__ballot(f >= (uint64_t)(p.flim / (uint32_t)W)) == 0) {
             for (int r = 0; r < nrs; ++r) {
                 const uint32_t len = TC[p.oFRm + r];
                 const uint32_t sp = SPI[r * W] & 0xffffu;
                 if (sp < (uint32_t)p.S) {
-                    int32_t x = X[sp], any = 0;
+                    uint32_t x = (uint32_t)X[sp], any = 0u;
                     uint32_t en[4];
                     if (kAhead && len > 0) gentries<W>(F, 0u, en);
                     for (uint32_t k = 0; k < len; k += 4) {   // len is a multiple of 4; padding adds 0
@@ -1116,12 +1117,12 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
                         for (int i = 0; i < 4; ++i) kc[i] = *reinterpret_cast<const int32_t*>(Kb + (e[i] & 0xffffu));
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            x = __mul24((int)(int16_t)(e[i] >> 16), kc[i]) + x;
+                            x = (uint32_t)__mul24((int)(int16_t)(e[i] >> 16), kc[i]) + x;
                             any |= x;
                         }
                     }
-                    X1[sp] = x;
-                    bad = bad || any < 0;
+                    X1[sp] = (int32_t)x;
+                    bad = bad || (any >> 31) != 0u;
                 }
                 F += len * W;
             }
