@@ -851,6 +851,8 @@ __device__ __forceinline__ void gentries(const uint32_t* E, uint32_t k, uint32_t
     asm volatile("" ::: "memory");
 }
 
+constexpr int LEAP_ATTEMPTS = 300;       // halvings after which a rejected leap gives up
+
 // One adaptive leap attempt (PreCalculations, T.cu:1568-2093).
 template <int G, int W, int PFM = 3>
 __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V, int l,
@@ -1159,6 +1161,11 @@ __device__ __forceinline__ int gleap(const KParams& p, GLane& L, const GView& V,
         gsync();
         CTL_PHASE(PH_UPDATE);
         if (!any_bad) break;
+        // 277 halvings bring any tau to 0, which draws nothing, so counts within
+        // [0, 2^31) pass by then.  A species that wrapped in an SSA step, or
+        // was given as 2^31 or more, fails whatever is drawn: only an SSA burst
+        // moves on.  (Counting this as a switch here cost 2 % at W = 64.)
+        if (__builtin_expect(attempt == LEAP_ATTEMPTS, 0)) return LEAP_SWITCH;
         tau = tau * 0.5f;
     }
     // check_time_instant (T.cu:1507-1562), per sampled species

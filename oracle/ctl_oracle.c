@@ -972,6 +972,8 @@ static int g_leap(grpctx* q) {
             s->X1[sp] = (int32_t)x;
         }
         if (ok) break;
+        /* tau is 0 by now: a species below 0 rejects whatever is drawn */
+        if (attempt == 300) { s->mode = MODE_SSA; return LEAP_SWITCH; }
         tau = tau * 0.5f;
     }
     leap_samples(s, (double)tau);

@@ -51,3 +51,27 @@ def test_firings_beyond_the_32_bit_sums(gpu, oracle_lib, G, n, geom):
         sim.run()
         _compare(sim, out, st, xf)
     m.close()
+
+
+@pytest.mark.parametrize("G,geom", [(2, {"slots": 12}), (4, {"slots": 12}), (16, {}), (64, {}), (8, {"compact_interval": 2})])
+def test_runs_with_a_count_above_the_top_end(gpu, oracle_lib, G, geom):
+    """A count of 2^31 or more runs as a negative one: no leap can be accepted (a species below 0 rejects whatever is
+    drawn), so every attempt has to give up for an SSA burst."""
+    print(f"case: above the top G={G} {geom}", flush=True)
+    left, right = [[1, 0, 0], [0, 1, 0], [1, 0, 0]], [[0, 1, 0], [1, 0, 0], [1, 0, 1]]
+    c, ts = [[1.0, 1.0, 1e-6]], np.array([0.5, 1.0])
+    x0 = np.array([[3000, 3000, 2**31 + 7], [3000, 3000, 10]], np.uint32)
+    out, st, xf = oracle_lib.run(left, right, x0.repeat(6, axis=0), c, ts, n=12, seed=1, final=True, group=G)
+    assert st["leaps"][:6].max() == 0 and st["rejections"][:6].min() > 100 and st["leaps"][6:].min() > 0
+    m = gpu.Model.from_arrays(left, right, x0.repeat(6, axis=0), c, ts)
+    with gpu.Sim(m, 12, 1, seed=1, lanes_per_sim=G, **geom) as sim:
+        sim.run()
+        _compare(sim, out, st, xf)
+    m.close()
+    models = [gpu.Model.from_arrays(left, right, x, c, ts) for x in x0]
+    with gpu.Batch(models, [6, 6], seed=1, lanes_per_sim=G) as b:
+        b.run()
+        for i in range(2):
+            assert np.array_equal(b.samples(i), out[6 * i:6 * i + 6])
+    for m in models:
+        m.close()
