@@ -429,12 +429,13 @@ int ctl_batch_create_lanes(const ctl_model* const* models, const int64_t* replic
         if ((rc = balloc(b, &c.d_done, 1))) return bail(rc);
         int maxS = 0, maxR = 0;
         size_t gwords = 0;
-        bool any_rates = false;
+        bool any_rates = false, plain = true;
         for (int i : c.models) {
             const ctl::Model& m = models[i]->m;
             maxS = std::max(maxS, m.S);
             maxR = std::max(maxR, m.R);
             any_rates = any_rates || m.c_rows != 1;
+            plain = plain && ctl::plain_values(m);
             if (c.G > 1) gwords = std::max(gwords, ctl::group_lds_words(m.S, m.R, c.G));
         }
         int per_cu = 0;
@@ -489,10 +490,10 @@ int ctl_batch_create_lanes(const ctl_model* const* models, const int64_t* replic
             g.iters = o->iters_per_launch > 0 ? o->iters_per_launch : 65536;
         } else {
             // the widest W at which every replica of the class is resident at
-            // once, as ctl_sim_create chooses it for one model; an explicit
-            // slot count keeps W = G
+            // once; an explicit slot count and models with negative rate
+            // constants or counts (plain_values) keep W = G
             c.W = c.G;
-            for (int w = 64; o->slots <= 0 && w > c.G && w >= 32; w /= 2) {
+            for (int w = 64; plain && o->slots <= 0 && w > c.G && w >= 32; w /= 2) {
                 int cu = 0;
                 e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&cu, ctl::gclass_kernel_fn(c.G, w), 64,
                                                                  (size_t)(64 / w) * gwords * 4);

@@ -1825,14 +1825,14 @@ inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, in
     }
     // change entries as byte offset of Kc[reaction] (R <= 8191: a group's LDS
     // holds 16384 words) | change << 16; flim: firings of a leap below which
-    // the update's sums fit 32 bits
+    // the update's sums fit 32 bits (0: never, a count may be negative)
     std::vector<uint32_t> fent(FSent.size());
     int vmax = 1;
     for (size_t h = 0; h < FSent.size(); ++h) {
         vmax = std::max(vmax, std::abs((int)(int16_t)(FSent[h] >> 16)));
         fent[h] = (FSent[h] & 0xffff0000u) | (FSent[h] & 0xffffu) * 4u;
     }
-    p.flim = std::min(1u << 23, (1u << 30) / (uint32_t)vmax);
+    p.flim = plain_values(m) ? std::min(1u << 23, (1u << 30) / (uint32_t)vmax) : 0u;
     rounds(W, sorder, FSptr, fent, p.oFRm, p.oFRe, 4, 0, 0u);
 }
 

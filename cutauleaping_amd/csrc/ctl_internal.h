@@ -57,6 +57,13 @@ struct Model {
 
 int compile_model(Model& m);   // validates and fills the compiled tables
 
+// Whether every rate constant is at least 0 and every initial and feed count
+// below 2^31, so that propensities are never negative.  The kernels keep a
+// propensity's critical flag in its sign bit; those that also sum propensities
+// from there (small_kernel, the group kernels' wider teams) run plain models
+// only.
+bool plain_values(const Model& m);
+
 }  // namespace ctl
 
 struct ctl_sim;

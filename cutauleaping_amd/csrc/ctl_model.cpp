@@ -121,6 +121,15 @@ int read_matrix_int(const std::string& path, int S_expected, std::vector<int32_t
 
 }  // namespace
 
+bool plain_values(const Model& m) {
+    uint32_t top = 0;
+    for (uint32_t x : m.x0) top |= x;
+    for (uint32_t x : m.fv) top |= x;
+    bool rates = true;
+    for (double c : m.c) rates = rates && c >= 0.0;
+    return rates && (top >> 31) == 0u;
+}
+
 int compile_model(Model& m) {
     const int S = m.S, R = m.R;
     if (S <= 0 || R <= 0) return fail(CTL_E_ARGS, "model needs at least one species and one reaction");

@@ -588,6 +588,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
     if (G < 1 || G > 64 || (G & (G - 1)))
         return bail(ctl::fail(CTL_E_ARGS, "lanes_per_sim must be 0 or a power of two up to 64"));
     s->lanes = G;
+    const bool plain = plain_values(m);
     int per_cu = 0;
     std::vector<uint32_t> small_tab;         // small_kernel's table (empty: not used)
     if (G > 1) {
@@ -638,9 +639,10 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         // At most 16 in force-SSA mode: an SSA step is one chain of selection
         // and update that a wider team does not shorten (cascade of 13 stages,
         // force-SSA: n = 5003 4.7 / 4.1 / 4.5 / 9.3).  An explicit geometry
-        // (block_size, slots, a regrouping interval) keeps W = G.
+        // (block_size, slots, a regrouping interval) keeps W = G, and so do
+        // negative rate constants and counts (plain_values).
         int W = G;
-        if (o->slots <= 0 && o->block_size <= 0 && o->compact_interval <= 0)
+        if (plain && o->slots <= 0 && o->block_size <= 0 && o->compact_interval <= 0)
             for (int w = o->force_ssa ? 16 : 64; w > G && w >= 16; w /= 2) {
                 const size_t sm = (size_t)(64 / w) * gwords * 4;
                 int cu = 0;
@@ -688,10 +690,10 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         }
         s->compact = compact > 0 && s->block > 64 ? compact : 0;
         // The default geometry of an LDS model runs small_kernel where the model
-        // is eligible; an explicit workgroup size or regrouping interval runs
-        // tau_leap_kernel.
+        // is eligible; an explicit workgroup size or regrouping interval and
+        // negative rate constants or counts (plain_values) run tau_leap_kernel.
         s->lpw = s->block;
-        if (s->lds && o->block_size == 0 && compact <= 0 && o->nc < (1 << 24)) {
+        if (plain && s->lds && o->block_size == 0 && compact <= 0 && o->nc < (1 << 24)) {
             small_tab = small_table(m, Dptr, Dent, &s->kp.oSD, &s->kp.snf);
             if (!small_tab.empty()) {
                 s->small = true;

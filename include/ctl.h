@@ -51,7 +51,9 @@ typedef struct {
     const int32_t* left;       /* R*S row-major [r][s], >= 0 (left_side) */
     const int32_t* right;      /* R*S row-major [r][s], >= 0 (right_side) */
     const int32_t* feed;       /* S flags, non-zero = feed-locked (M_feed); NULL = none */
-    const uint32_t* x0;        /* x0_rows * S initial counts (MX_0 rows) */
+    const uint32_t* x0;        /* x0_rows * S initial counts (MX_0 rows); counts are kept
+                                  as int32: 2^31 and more are accepted, as initial counts
+                                  and as feeds, but run as negative numbers */
     int64_t x0_rows;           /* 1: shared by every simulation; >= n: one row per
                                   simulation (the reference); otherwise n/x0_rows
                                   consecutive simulations share a row (replicas) */
