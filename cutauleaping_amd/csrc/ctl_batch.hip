@@ -646,9 +646,14 @@ int ctl_batch_run(ctl_batch* b) {
         BHIP(hipMemsetAsync(c.d_done, 0, sizeof(uint32_t), c.stream), "memset");
         c.finished = false;
     }
-    // replica counters of every model (before any class starts)
-    BHIP(hipMemset(b->d_rep_next, 0, sizeof(uint32_t) * b->nmodels), "memset");
-    BHIP(hipMemset(b->d_tot, 0, ST_COUNT * sizeof(*b->d_tot)), "memset");
+    // Replica counters of every model, before any class starts.  The classes'
+    // streams do not wait for the null stream, so the first class's stream
+    // clears them and the others wait for it.
+    hipStream_t st0 = b->classes[0].stream;
+    BHIP(hipMemsetAsync(b->d_rep_next, 0, sizeof(uint32_t) * b->nmodels, st0), "memset");
+    BHIP(hipEventRecord(b->classes[0].ev0, st0), "hipEventRecord");
+    for (size_t k = 1; k < b->classes.size(); ++k)
+        BHIP(hipStreamWaitEvent(b->classes[k].stream, b->classes[0].ev0, 0), "hipStreamWaitEvent");
     ctl_stats& S = b->stats;
     S.launches = 0;
     // The classes run concurrently: each round launches every unfinished
@@ -698,7 +703,7 @@ int ctl_batch_run(ctl_batch* b) {
     }
     S.kernel_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - k0).count();
     unsigned long long tot[ST_COUNT];
-    hipStream_t st0 = b->classes[0].stream;
+    BHIP(hipMemsetAsync(b->d_tot, 0, ST_COUNT * sizeof(*b->d_tot), st0), "memset");
     hipLaunchKernelGGL(batch_stat_kernel, dim3(b->nmodels), dim3(STAT_BLOCK), 0, st0, b->d_desc, b->d_tot);
     BHIP(hipGetLastError(), "batch_stat_kernel launch");
     BHIP(hipMemcpyAsync(tot, b->d_tot, sizeof tot, hipMemcpyDeviceToHost, st0), "hipMemcpy D2H");

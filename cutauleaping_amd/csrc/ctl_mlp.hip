@@ -998,7 +998,8 @@ int ctl_mlp_create(const int32_t* widths, int32_t nlayers, int32_t gpu, uint64_t
         for (long i = 0; i < (long)widths[l] * widths[l + 1]; ++i) h[n->woff[l] + i] = U(rng);
     }
     if ((e = hipMemcpy(n->w, h.data(), sizeof(float) * off, hipMemcpyHostToDevice)) != hipSuccess) return bail(mfail(e, "H2D"));
-    if ((e = hipMemset(n->m, 0, sizeof(float) * off)) != hipSuccess || (e = hipMemset(n->v, 0, sizeof(float) * off)) != hipSuccess)
+    if ((e = hipMemsetAsync(n->m, 0, sizeof(float) * off, n->stream)) != hipSuccess ||
+        (e = hipMemsetAsync(n->v, 0, sizeof(float) * off, n->stream)) != hipSuccess)
         return bail(mfail(e, "memset"));
     refresh_bf16(n);
     if ((e = hipStreamSynchronize(n->stream)) != hipSuccess) return bail(mfail(e, "init"));
