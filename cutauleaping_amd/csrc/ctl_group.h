@@ -1532,10 +1532,14 @@ __device__ __forceinline__ bool gregroup(int key, int reg, uint32_t* cnt, uint32
 // Waves per SIMD the group kernels are compiled for.  W = G: G = 8, 16 and 32
 // for four (128 VGPRs, a few bytes of scratch), measured +9 % at G = 16 and
 // +4 % at G = 32 on the 100x200 network, +24 % at G = 8 on the 50x100 sweep
-// network; G = 4 groups are bounded by LDS instead, and G = 64 would spill
-// heavily.  W > G serves runs that leave the chip short of wavefronts.
-__host__ __device__ constexpr int gwaves(int G, int W) {
-    return W > G ? (W == 64 ? 2 : 4) : (G == 8 || G == 16 || G == 32 ? 4 : 1);
+// network; G = 64 would spill heavily.  G = 2 and 4 hold three by themselves
+// except in mode 1 (174 VGPRs, where three waves have 168 each): two spilled
+// registers there give the third wave back (14 species and 40 reactions,
+// 262144 simulations, two / three: adaptive 35.6 / 26.4 ms, force-SSA
+// 29.6 / 21.0; larger models are bounded by LDS).  W > G serves runs that
+// leave the chip short of wavefronts.
+__host__ __device__ constexpr int gwaves(int G, int W, int PFM = 3) {
+    return W > G ? (W == 64 ? 2 : 4) : (G == 8 || G == 16 || G == 32 ? 4 : (G <= 4 && PFM == 1 ? 3 : 1));
 }
 
 // Persistent group kernel: p.ns lanes = p.ns / W group slots, each pulling
@@ -1547,7 +1551,7 @@ __host__ __device__ constexpr int gwaves(int G, int W) {
 // running has switched, so that bursts run side by side.  Either way each simulation's events and draws are its own;
 // only the order in which the lanes serve the simulations moves.
 template <int G, int W, bool RG, int PF>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gwaves(G, W)))) void group_kernel(KParams p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gwaves(G, W, PF)))) void group_kernel(KParams p) {
     extern __shared__ uint32_t smem[];
     __shared__ float recip[64];
     __shared__ uint32_t rg_cnt[12];
@@ -1709,6 +1713,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gwaves(G, W
     CTL_PHASE_FLUSH();
 }
 
+// Host: propensity mode (pmode) of a model at G lanes: with at most two
+// reactant entries of multiplicity <= 2 per reaction, two table entries per
+// reaction -- factor indices (1) when the factor table fits in the Kc region,
+// free outside the count and update phases, else species | multiplicity read
+// from the state (2): a separate table would enlarge every group's LDS and
+// cost occupancy (the enzyme cascade, 61 species and 60 reactions at G = 4,
+// ran 20 % slower with one).
+inline int group_pmode(const Model& m, int G) {
+    bool two = true;
+    for (int j = 0; j < m.R; ++j) {
+        if (m.Lptr[j + 1] - m.Lptr[j] > 2) two = false;
+        for (uint32_t h = m.Lptr[j]; h < m.Lptr[j + 1]; ++h)
+            if ((m.Lent[h] >> 16) > 2) two = false;
+    }
+    return !two ? 0 : (2 * m.S + 1 <= group_rpad(m.R, G) ? 1 : 2);
+}
+
 // Host: appends the lane-interleaved round streams (KParams::oPRm ..) of a
 // group kernel with G lanes to the packed table buffer T.
 inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, int W, const Model& m,
@@ -1739,20 +1760,7 @@ inline void append_group_streams(std::vector<uint32_t>& T, KParams& p, int G, in
         oe = (int)T.size();
         T.insert(T.end(), e.begin(), e.end());
     };
-    // propensity mode (pmode): with at most two reactant entries of
-    // multiplicity <= 2 per reaction, two table entries per reaction -- factor
-    // indices (1) when the factor table fits in the Kc region, free outside
-    // the count and update phases, else species | multiplicity read from the
-    // state (2): a separate table would enlarge every group's LDS and cost
-    // occupancy (the enzyme cascade, 61 species and 60 reactions at G = 4,
-    // ran 20 % slower with one)
-    bool two = true;
-    for (int j = 0; j < m.R; ++j) {
-        if (m.Lptr[j + 1] - m.Lptr[j] > 2) two = false;
-        for (uint32_t h = m.Lptr[j]; h < m.Lptr[j + 1]; ++h)
-            if ((m.Lent[h] >> 16) > 2) two = false;
-    }
-    p.pfast = !two ? 0 : (2 * m.S + 1 <= group_rpad(m.R, G) ? 1 : 2);
+    p.pfast = group_pmode(m, G);
     std::vector<int> rorder((size_t)((m.R + G - 1) / G) * G, -1);
     for (int j = 0; j < m.R; ++j) rorder[j] = j;          // reaction j: lane j mod G (the selection's partials)
     // pfast: a reactant entry becomes its index in the factor table F

@@ -593,6 +593,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
     std::vector<uint32_t> small_tab;         // small_kernel's table (empty: not used)
     if (G > 1) {
         const size_t gwords = group_lds_words(S, R, G);    // group LDS words per simulation
+        const int pf = group_pmode(m, G);
         if (gwords * 4 > 65536) return bail(ctl::fail(CTL_E_LIMIT, "model too large for the group kernel (more than 64 KB of LDS)"));
         // Regrouping simulations by mode (leap / SSA) every `compact` iterations
         // is done on request only: a wavefront whose groups are in both modes
@@ -646,7 +647,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
             for (int w = o->force_ssa ? 16 : 64; w > G && w >= 16; w /= 2) {
                 const size_t sm = (size_t)(64 / w) * gwords * 4;
                 int cu = 0;
-                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&cu, group_kernel_fn(G, w, false, 1), 64, sm);
+                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&cu, group_kernel_fn(G, w, false, pf), 64, sm);
                 const long long need = w < 64 && R <= 14 * G ? n + (long long)n / 3 : n;
                 if (e == hipSuccess && (long long)prop.multiProcessorCount * cu * (64 / w) >= need) {
                     W = w;
@@ -659,7 +660,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         s->smem = (size_t)gpb * gwords * 4;
         s->lds = true;
         s->compact = compact > 0 && W == G && G < 64 && s->block > 64 ? compact : 0;
-        const void* kfn = group_kernel_fn(G, W, s->compact > 0, 1);   // occupancy (the instances alike)
+        const void* kfn = group_kernel_fn(G, W, s->compact > 0, pf);
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, s->block, s->smem);
         if (e != hipSuccess || per_cu <= 0) per_cu = 1;
         long long groups = o->slots > 0 ? (long long)o->slots : (long long)prop.multiProcessorCount * per_cu * gpb;
