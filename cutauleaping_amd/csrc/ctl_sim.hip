@@ -697,22 +697,62 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         if (plain && s->lds && o->block_size == 0 && compact <= 0 && o->nc < (1 << 24)) {
             small_tab = small_table(m, Dptr, Dent, &s->kp.oSD, &s->kp.snf);
             if (!small_tab.empty()) {
-                s->small = true;
-                s->smem = (small_tab.size() + (m.c_rows == 1 ? R : 0)) * 4 +
-                          (size_t)small_words(S, R, s->kp.snf, m.c_rows == 1) * 4 * 64;
+                const long long cus = prop.multiProcessorCount;
+                auto small_smem = [&](int lpw) {
+                    return (small_tab.size() + (m.c_rows == 1 ? R : 0)) * 4 +
+                           (size_t)small_words(S, R, s->kp.snf, m.c_rows == 1) * 4 * lpw;
+                };
+                auto waves_per_cu = [&](const void* fn, size_t smem) {
+                    int cu = 0;
+                    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&cu, fn, 64, smem) == hipSuccess ? cu : 0;
+                };
                 // Lanes of a wavefront that hold a simulation: 64 when the
                 // simulations fill the chip, and in force-SSA mode, where the
-                // lanes of a wavefront run in step; adaptive runs with up to
-                // two simulations per resident wavefront spread out, since
-                // leaps and SSA bursts of one wavefront's lanes run one after
-                // the other.  Schlogl to t = 10, kernel ms at 1 / 2 / 8 / 64
-                // lanes: n = 1024 52 / 60 / 62 / 79, n = 4096 56 / 62 / 76 /
-                // 81; to t = 2.5, n = 16384 (8 / 64) 21.3 / 21.0; force-SSA to
-                // t = 1, n = 4096: 9.7 / 8.4 / 8.6 / 7.7.
-                const long long waves = (long long)prop.multiProcessorCount * 16;
-                if (!o->force_ssa && o->slots <= 0 && n <= 2 * waves) s->lpw = n <= waves ? 1 : 2;
-                s->smem = (small_tab.size() + (m.c_rows == 1 ? R : 0)) * 4 +
-                          (size_t)small_words(S, R, s->kp.snf, m.c_rows == 1) * 4 * s->lpw;
+                // lanes of a wavefront run in step; small adaptive runs spread
+                // out to 1 or 2, since leaps and SSA bursts of one wavefront's
+                // lanes run one after the other, where all their wavefronts
+                // are resident (the table is per wavefront: 2 species and 58
+                // reactions hold 10 a CU, n = 4096 at 1 / 2 lanes: 180 / 101
+                // ms).  Schlogl to t = 10, kernel ms at 1 / 2 / 8 / 64 lanes:
+                // n = 1024 52 / 60 / 62 / 79, n = 4096 56 / 62 / 76 / 81; to
+                // t = 2.5, n = 16384 (8 / 64) 21.3 / 21.0; force-SSA to t = 1,
+                // n = 4096: 9.7 / 8.4 / 8.6 / 7.7.
+                // With more than two species per reaction a leap's rebuild of
+                // the factors outweighs the divergence once wavefronts of a CU
+                // slow each other: at 3 to 6 of them, and above 12; with 5
+                // factors a species above 2 at all.  Leaps of 16 species and 4
+                // reactions, ms at 512 / 1024 / 2048 / 4096 wavefronts of one
+                // lane 2.9 / 3.8 / 2.8 / 3.8, of 64 lanes 3.7; 28 species and
+                // 6 reactions of order 3: 6.2 / 8.2 / 6.1 / 7.9, 64 lanes 6.1.
+                const bool heavy = S > 2 * R;
+                if (!o->force_ssa && o->slots <= 0)
+                    for (int w = 1; w <= (!heavy ? 2 : s->kp.snf == 2 ? 4 : 1) && s->lpw == 64; w *= 2) {
+                        const long long waves = ((long long)n + w - 1) / w;
+                        const bool eased = waves <= 2 * cus ||
+                                           (s->kp.snf == 2 && 2 * waves > 13 * cus && waves <= 12 * cus);
+                        if ((!heavy || eased) && waves <= cus * waves_per_cu(small_kernel_fn(R), small_smem(w))) s->lpw = w;
+                    }
+                // A simulation holds 1.5 to 3 times the words of
+                // tau_leap_kernel's, so fewer are resident.  While all of them
+                // are (or as many as of tau_leap_kernel's) this kernel is the
+                // faster one.  Beyond, its SSA step still is, except with few
+                // reactions to a simulation's words, and its leaps are not:
+                // their rebuild of the factors grows with the species.
+                // Kernel ms, this / tau_leap_kernel (wavefronts a CU):
+                //   8 species, 44 reactions (6 / 10), n = 131072   leaps 48 % more, mixed 0.51 times
+                //   14 species, 14 reactions (8 / 14), n = 393216  leaps 26 % more, mixed 0.48 times
+                //   16 species, 30 reactions (6 / 9), n = 131072   leaps 129 / 83, mixed 109 / 158
+                //   18 species, 28 reactions (5 / 9), n = 131072   leaps 59 % more, mixed 23 % more
+                //   20 species, 20 reactions of order 3 (3 / 10), n = 131072  leaps 87 / 35, mixed 27 / 30
+                //   28 species, 6 reactions of order 3 (3 / 9), n = 131072    leaps 18.5 / 5.8, force-SSA 2.4 / 1.3
+                //   20 species, 20 reactions (5 / 10), n = 131072  force-SSA 0.68 times
+                const long long held = o->slots > 0 ? std::min((long long)n, (long long)o->slots) : n;
+                const int own = waves_per_cu(small_kernel_fn(R), small_smem(64));
+                const int other = waves_per_cu((const void*)tau_leap_kernel<true>, s->smem);
+                s->small = s->lpw < 64 || held <= cus * own * 64 || own >= other ||
+                           (o->force_ssa ? S <= 2 * R || own >= 8 : S <= 14);
+                if (s->small) s->smem = small_smem(s->lpw);
+                else small_tab.clear();
             }
         }
         const void* kfn = s->small ? small_kernel_fn(R) : s->lds ? (const void*)tau_leap_kernel<true> : (const void*)tau_leap_kernel<false>;
