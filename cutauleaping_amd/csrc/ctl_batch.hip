@@ -297,7 +297,7 @@ int upload_model(ctl_batch* b, const ctl::Model& m, KParams& p, int G, int W) {
     }
     std::vector<float> cf(m.c.size());
     for (size_t i = 0; i < m.c.size(); ++i) cf[i] = (float)m.c[i];
-    uint32_t *Lptr, *Lent, *Fptr, *Fent, *Vptr, *Vent, *Dp, *De, *hw, *x0, *FSp, *FSe;
+    uint32_t *Lptr, *Lent, *Fptr, *Fent, *Vptr, *Vent, *Dp, *De, *hw, *x0;
     int32_t* cs;
     double* ts;
     float* cdev;
@@ -308,11 +308,8 @@ int upload_model(ctl_batch* b, const ctl::Model& m, KParams& p, int G, int W) {
         (rc = bupload(b, &Dp, Dptr.data(), Dptr.size())) || (rc = bupload(b, &De, Dent.data(), Dent.size())) ||
         (rc = bupload(b, &hw, horw.data(), horw.size())) || (rc = bupload(b, &cs, m.cs.data(), m.cs.size())) ||
         (rc = bupload(b, &ts, m.ts.data(), m.ts.size())) || (rc = bupload(b, &cdev, cf.data(), cf.size())) ||
-        (rc = bupload(b, &x0, m.x0.data(), m.x0.size())) ||
-        (rc = bupload(b, &FSp, FSptr.data(), FSptr.size())) || (rc = bupload(b, &FSe, FSent.data(), FSent.size())))
+        (rc = bupload(b, &x0, m.x0.data(), m.x0.size())))
         return rc;
-    p.FSptr = FSp;
-    p.FSent = FSe;
     p.nfs = (int)m.fs.size();
     p.fs = nullptr;
     p.fv = nullptr;
@@ -329,14 +326,7 @@ int upload_model(ctl_batch* b, const ctl::Model& m, KParams& p, int G, int W) {
         auto put = [&](const uint32_t* d, size_t k) { const int o = (int)T.size(); T.insert(T.end(), d, d + k); return o; };
         p.oLp = put(m.Lptr.data(), m.Lptr.size());
         p.oLe = put(m.Lent.data(), m.Lent.size());
-        p.oVp = put(m.Vptr.data(), m.Vptr.size());
-        p.oVe = put(m.Vent.data(), m.Vent.size());
-        p.oHw = put(horw.data(), horw.size());
-        p.oFSp = put(FSptr.data(), FSptr.size());
-        p.oFSe = put(FSent.data(), FSent.size());
-        p.oFp = put(m.Fptr.data(), m.Fptr.size());
         p.oFe = put(m.Fent.data(), m.Fent.size());
-        p.oDp = put(Dptr.data(), Dptr.size());
         p.oDe = put(Dent.data(), Dent.size());
         p.oCs = put(reinterpret_cast<const uint32_t*>(m.cs.data()), m.cs.size());
         if (G > 1) append_group_streams(T, p, G, W, m, FSptr, FSent, Dptr, Dent);

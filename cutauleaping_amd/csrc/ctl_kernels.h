@@ -59,24 +59,23 @@ struct KParams {
     const uint32_t* Vent;
     const uint32_t* Dptr;     // SSA dependency graph: reactions whose propensity
     const uint32_t* Dent;     //   reads a species changed by reaction j
-    const uint32_t* FSptr;    // fear entries species-major, ascending reaction
-    const uint32_t* FSent;    //   (group kernel's per-species update)
     // The u32 tables packed in one buffer, each at a 32-bit word offset: the
     // group kernels address every table from one base pointer, which keeps
     // their scalar-register footprint small.
     const uint32_t* T;
-    int oLp, oLe, oVp, oVe, oHw, oFSp, oFSe, oFp, oFe, oDp, oDe, oCs;
-    // Lane-interleaved round streams of the group kernel, built for its G:
-    // round r covers reactions (or species) r*G .. r*G+G-1, lane l takes the
-    // r*G+l-th; the round holds len = T[o*m + r] entries per lane, entry k of
-    // lane l at T[o*e + base_r + k*G + l] (base_r = G * sum of the earlier
-    // lengths).  Shorter lists are padded with 0 (multiplicity / change 0);
-    // var and fear round lengths are multiples of 4 (loads issue 4 at a time).
+    int oLp, oLe, oFe, oDe, oCs;
+    // Lane-interleaved round streams of the group kernel.  A round of B lanes
+    // (B = G for the reactant rounds, W for the species ones) covers reactions
+    // (or species) r*B .. r*B+B-1, lane l takes the r*B+l-th; the round holds
+    // len = T[o*m + r] entries per lane, entry k of lane l at
+    // T[o*e + base_r + k*B + l] (base_r = B * sum of the earlier lengths).
+    // Shorter lists are padded with 0 (multiplicity / change 0); var and fear
+    // round lengths are multiples of 4 (loads issue 4 at a time).
     // Reactant entries (species | multiplicity << 16; with pfast the index of
     // the reactant's factor in the group's factor table, padding 2S), var
     // entries of the tau' sums and species-major fear entries (byte offset of
     // the reaction's count | change << 16).
-    // Var and fear rounds list species in the order T[oSPI + r*G + l]
+    // Var and fear rounds list species in the order T[oSPI + r*W + l]
     // (species | HOR << 16 | HORtype << 24; 0xffffffff: none), longest lists
     // first.  gsimple: no species has HOR 3 or HOR 2 of type 2, so g is 1 or 2.
     int oPRm, oPRe, oVRm, oVRe, oFRm, oFRe, oSPI, gsimple;
@@ -93,7 +92,7 @@ struct KParams {
     // Small models (small_kernel): words T[oST .. oST + nST), copied to LDS at
     // the start of a launch (layout: ctl_small.h); nST = 0: not eligible.
     int oST, nST, oSD;        // oSD: first word of the dependents in the table
-    int snf;                  // factor words per species (2, or 4 with a multiplicity of 3)
+    int snf;                  // factor words per species (2, or 5 with a multiplicity of 3)
     const uint32_t* horw;     // hor | hort << 8
     const int32_t* cs;
     const double* ts;

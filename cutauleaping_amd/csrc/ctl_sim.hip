@@ -786,7 +786,7 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
                 FSent[cnt[e & 0xffffu]++] = (uint32_t)j | (e & 0xffff0000u);
             }
     }
-    uint32_t *Lptr, *Lent, *Fptr, *Fent, *Vptr, *Vent, *Dp, *De, *hw, *FSp, *FSe;
+    uint32_t *Lptr, *Lent, *Fptr, *Fent, *Vptr, *Vent, *Dp, *De, *hw;
     int32_t* cs;
     double* ts;
     if ((rc = upload(s, &Lptr, m.Lptr.data(), m.Lptr.size())) || (rc = upload(s, &Lent, m.Lent.data(), m.Lent.size())) ||
@@ -794,24 +794,14 @@ int ctl_sim_create(const ctl_model* mh, const ctl_opts* o, ctl_sim** out) {
         (rc = upload(s, &Vptr, m.Vptr.data(), m.Vptr.size())) || (rc = upload(s, &Vent, m.Vent.data(), m.Vent.size())) ||
         (rc = upload(s, &Dp, Dptr.data(), Dptr.size())) || (rc = upload(s, &De, Dent.data(), Dent.size())) ||
         (rc = upload(s, &hw, horw.data(), horw.size())) || (rc = upload(s, &cs, m.cs.data(), m.cs.size())) ||
-        (rc = upload(s, &ts, m.ts.data(), m.ts.size())) ||
-        (rc = upload(s, &FSp, FSptr.data(), FSptr.size())) || (rc = upload(s, &FSe, FSent.data(), FSent.size())))
+        (rc = upload(s, &ts, m.ts.data(), m.ts.size())))
         return bail(rc);
-    p.FSptr = FSp;
-    p.FSent = FSe;
     {   // the same tables packed behind one base pointer (group kernels)
         std::vector<uint32_t> T;
         auto put = [&](const uint32_t* d, size_t k) { const int o = (int)T.size(); T.insert(T.end(), d, d + k); return o; };
         p.oLp = put(m.Lptr.data(), m.Lptr.size());
         p.oLe = put(m.Lent.data(), m.Lent.size());
-        p.oVp = put(m.Vptr.data(), m.Vptr.size());
-        p.oVe = put(m.Vent.data(), m.Vent.size());
-        p.oHw = put(horw.data(), horw.size());
-        p.oFSp = put(FSptr.data(), FSptr.size());
-        p.oFSe = put(FSent.data(), FSent.size());
-        p.oFp = put(m.Fptr.data(), m.Fptr.size());
         p.oFe = put(m.Fent.data(), m.Fent.size());
-        p.oDp = put(Dptr.data(), Dptr.size());
         p.oDe = put(Dent.data(), Dent.size());
         p.oCs = put(reinterpret_cast<const uint32_t*>(m.cs.data()), m.cs.size());
         if (s->lanes > 1) append_group_streams(T, p, s->lanes, s->width, m, FSptr, FSent, Dptr, Dent);

@@ -24,7 +24,7 @@ __device__ __forceinline__ void stat_add(const ctl_sim_stat* __restrict__ st, in
                                          unsigned long long* tot) {
     __shared__ unsigned long long part[STAT_BLOCK / 64][ST_COUNT];
     unsigned long long v[ST_COUNT] = {};
-    for (int i = first; i < n; i += stride) {
+    for (long i = first; i < n; i += stride) {        // past n by up to a stride: not an int's sum
         const ctl_sim_stat x = st[i];
         v[ST_FIRINGS] += x.firings;
         v[ST_LEAPS] += x.leaps;
