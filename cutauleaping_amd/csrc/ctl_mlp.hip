@@ -37,6 +37,7 @@ namespace ctl {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint16_t f2bf(float f) {
     uint32_t u = __float_as_uint(f);
@@ -269,7 +270,11 @@ __global__ __launch_bounds__(64) void gemm_frag(GemmArgs g) {
 // of rows): four wavefronts of 64 x 64, A and B staged in LDS in two slabs of
 // 32 k (rows padded to 40 elements), the next slab's loads in flight during
 // the products of the current one.  Fragments straight from memory are bound
-// by their 32-byte rows there (65536 x 1000 x 256: MEASUREDBIG).
+// by their 32-byte rows there (us by fragments / here, rows x k x columns:
+// 65536 x 2048 x 2048 2431 / 898, 612 TFLOP/s; 65536 x 288 x 1000 169 / 124;
+// at the line, 256 tiles, 8192 x 512 x 512 28.1 / 22.5; at half of it 4096 x
+// 512 x 512 16.7 / 20.5).  The pieces on their way are native vectors: as
+// HIP's uint4 they went through scratch memory, 2452 us for the largest.
 constexpr int GKP = 40;
 template <int EPI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_lds(GemmArgs g) {
@@ -299,11 +304,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         for (int c = 0; c < 2; ++c)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[a][c][v] = 0.0f;
-    uint4 ra[2], rb[2];
+    u32x4 ra[2], rb[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        ra[t] = *reinterpret_cast<const uint4*>(pa[t]);
-        rb[t] = *reinterpret_cast<const uint4*>(pb[t]);
+        ra[t] = *reinterpret_cast<const u32x4*>(pa[t]);
+        rb[t] = *reinterpret_cast<const u32x4*>(pb[t]);
     }
     const int slabs = g.K / 32;
     for (int s = 0; s < slabs; ++s) {
@@ -311,15 +316,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         uint16_t* const B = Bs[s & 1];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            *reinterpret_cast<uint4*>(A + sa[t]) = ra[t];
-            *reinterpret_cast<uint4*>(B + sa[t]) = rb[t];
+            *reinterpret_cast<u32x4*>(A + sa[t]) = ra[t];
+            *reinterpret_cast<u32x4*>(B + sa[t]) = rb[t];
         }
         __syncthreads();             // the other buffer's readers passed the previous barrier
         const int n = s + 1 < slabs ? s + 1 : s;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            ra[t] = *reinterpret_cast<const uint4*>(pa[t] + n * 32);
-            rb[t] = *reinterpret_cast<const uint4*>(pb[t] + n * bstep);
+            ra[t] = *reinterpret_cast<const u32x4*>(pa[t] + n * 32);
+            rb[t] = *reinterpret_cast<const u32x4*>(pb[t] + n * bstep);
         }
 #pragma unroll
         for (int ks = 0; ks < 32; ks += 16) {
