@@ -434,6 +434,15 @@ int ctl_batch_create_lanes(const ctl_model* const* models, const int64_t* replic
             e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)batch_kernel, c.block, 0);
             if (e != hipSuccess || per_cu <= 0) per_cu = 1;
             int ns = o->slots > 0 ? o->slots : prop.multiProcessorCount * per_cu * c.block;
+            // No more wavefronts than chunks (of 64 replicas of a model): with
+            // wavefronts to spare, those that come first take the chunks and
+            // some CUs serve several times what others do.  ms at 262144 slots
+            // / as many as the chunks fill: Schlogl, 65536 replicas 18.6 /
+            // 15.3, 131072 19.8 / 17.5; 16 species and 30 reactions, 131072
+            // 178 / 121.
+            long long chunks = 0;
+            for (int i : c.models) chunks += (replicas[i] + 63) / 64;
+            if (o->slots <= 0) ns = (int)std::min((long long)ns, chunks * 64);
             ns = ((ns + c.block - 1) / c.block) * c.block;
             c.ns = ns;
             c.grid = ns / c.block;

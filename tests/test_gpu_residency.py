@@ -45,3 +45,19 @@ def test_widths_around_the_residency_bit_exact(gpu, oracle_lib, S, R, order):
         s.run()
         _compare(s, *oracle_lib.run(left, right, x0, c, ts, n=n, seed=3, final=True, group=4))
     m.close()
+
+
+def test_a_batch_of_one_lane_models_has_a_wavefront_per_chunk(gpu, oracle_lib):
+    print("case: residency batch", flush=True)
+    cases = [_ring(5, 9, 1), _ring(7, 8, 1)]
+    x0, ts, reps = [np.full((1, S), 20, np.uint32) for S in (5, 7)], np.array([0.01, 0.02]), [65, 60001]
+    ms = [gpu.Model.from_arrays(l, r, x, c, ts) for (l, r, c), x in zip(cases, x0)]
+    with gpu.Batch(ms, reps, seed=3) as b:
+        b.run()
+        assert b.stats()["slots"] == -(-(2 + 938) * 64 // 256) * 256        # chunks of 64, workgroups of 256 lanes
+        for i, (l, r, c) in enumerate(cases):
+            assert b.model_lanes(i) == 1
+            out, _ = oracle_lib.run(l, r, x0[i], c, ts, n=reps[i], seed=3, sim_base=b.stream_base(i), threads=8)
+            assert np.array_equal(b.samples(i), out), i
+    for m in ms:
+        m.close()
