@@ -211,30 +211,31 @@ __global__ void to_reference_layout(const uint32_t* __restrict__ src, uint32_t* 
 // thread index within the group; mean over the P simulations at
 // (g*P + par)*threads + tid, then sum over samples, sampled species and
 // target repetitions of |tgt - mean| / tgt (tgt != 0), divided by K*SS.
-// One wavefront per value.  The FP32 sum is a chain in (sample, species,
-// repetition) order; what it adds is independent, so the 64 lanes work out 64
-// distances (P loads, one load, two divisions each) into LDS and lane 0 adds
-// them in that order.  One thread per value did all of it in the chain, one
-// memory latency after the other: 512 values of 300 distances over 8
-// repetitions 0.52 ms, now under 0.1 ms.
+// The FP32 sum is a chain in (sample, species, repetition) order; what it adds
+// is independent.  Two kernels; ctl_fitness chooses.
+//
+// fitness_kernel: one wavefront per value; the 64 lanes work out 64 distances
+// (P loads, one load, two divisions each) into LDS and lane 0 adds them in that
+// order.  total = K SS E distances, below 2^32.
 __global__ __launch_bounds__(64) void fitness_kernel(const uint32_t* __restrict__ samples,
                                                      const uint32_t* __restrict__ target,
                                                      const int8_t* __restrict__ t2e, double* __restrict__ fit,
                                                      int threads, size_t nf, int P, int K, int SS, int D, int E) {
     __shared__ double term[64];
-    const int l = threadIdx.x;
-    const size_t KS = (size_t)K * SS, total = KS * E;
+    const uint32_t l = threadIdx.x;
+    const size_t KS = (size_t)K * SS;
+    const uint32_t total = (uint32_t)(KS * E);
     for (size_t tid = blockIdx.x; tid < nf; tid += gridDim.x) {
         const size_t g = tid / threads, th = tid % threads;
         const int experiment = t2e[tid];
         const uint32_t* own = samples + (g * P * threads + th) * KS;
         float sub = 0.0f;
-        for (size_t q0 = 0; q0 < total; q0 += 64) {
-            const size_t q = q0 + l;
+        for (uint32_t q0 = 0; q0 < total; q0 += 64) {
+            const uint32_t q = q0 + l;
             double dist = 0.0;                   // past the end: adds an exact 0
             if (q < total) {
-                const size_t col = q / E;
-                const int i = (int)(col / SS), s = (int)(col % SS), rep = (int)(q % E);
+                const uint32_t col = q / (uint32_t)E, rep = q - col * (uint32_t)E;
+                const uint32_t i = col / (uint32_t)SS, s = col - i * (uint32_t)SS;
                 double acc = 0.0;
                 for (int par = 0; par < P; ++par) acc += own[(size_t)par * threads * KS + col];
                 acc /= P;
@@ -252,9 +253,36 @@ __global__ __launch_bounds__(64) void fitness_kernel(const uint32_t* __restrict_
                 }
             }
             __syncthreads();
+            if (total - q0 <= 64) break;         // q0 + 64 may pass 2^32
         }
         if (l == 0) fit[tid] = (1.0 / K) * (1.0 / SS) * sub;
     }
+}
+
+// One thread per value.
+__global__ __launch_bounds__(256) void fitness_each(const uint32_t* __restrict__ samples,
+                                                    const uint32_t* __restrict__ target,
+                                                    const int8_t* __restrict__ t2e, double* __restrict__ fit,
+                                                    int threads, size_t nf, int P, int K, int SS, int D, int E) {
+    const size_t tid = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (tid >= nf) return;
+    const size_t g = tid / threads, th = tid % threads, KS = (size_t)K * SS;
+    const uint32_t* own = samples + (g * P * threads + th) * KS;
+    const uint32_t* tg = target + (size_t)t2e[tid] * (SS * E);
+    float sub = 0.0f;
+    for (int i = 0; i < K; ++i, tg += (size_t)SS * D * E)
+        for (int s = 0; s < SS; ++s, ++own) {
+            double acc = 0.0;
+            for (int par = 0; par < P; ++par) acc += own[(size_t)par * threads * KS];
+            acc /= P;
+            for (int rep = 0; rep < E; ++rep) {
+                const int tgt = (int)tg[rep * SS + s];
+                double dist = fabs((double)tgt - acc);
+                if (tgt != 0) dist /= tgt;
+                sub += dist;
+            }
+        }
+    fit[tid] = (1.0 / K) * (1.0 / SS) * sub;
 }
 
 // Per-group moments of the samples in two passes.  Pass 1: the replicas of a
@@ -1028,9 +1056,25 @@ int ctl_fitness(const ctl_sim* sc, double* out, size_t count) {
     }
     if (!s->d_fit && (rc = dalloc(s, &s->d_fit, nf))) return rc;    // once per sim, reused by later calls
     double* d_fit = s->d_fit;
-    hipLaunchKernelGGL(fitness_kernel, dim3((unsigned)std::min<size_t>(nf, 1 << 20)), dim3(64), 0, s->stream,
-                       s->kp.storage, s->d_target, s->d_t2e, d_fit, threads, nf, P, s->kp.K, s->kp.SS, (int)f.experiments,
-                       (int)f.repetitions);
+    const size_t total = (size_t)s->kp.K * s->kp.SS * f.repetitions;
+    // A wavefront per value, except where a value is little work, or its row of
+    // samples one stream and the rows in progress fit the L2.  us of the call,
+    // wavefront / thread per value, at 512, 8192, 65536 and 524288 values:
+    //   P = 1, 3 distances     28 / 28   52 / 49   263 / 51    481 / 317
+    //          15              26 / 29   29 / 29    73 / 54    494 / 342
+    //          63              27 / 47   31 / 47    87 / 74    626 / 897
+    //          600             38 / 160  68 / 162  344 / 225  2587 / 2994
+    //   P = 8, 63              28 / 99   32 / 135  105 / 633   828 / 5413
+    const bool light = (size_t)P * s->kp.K * s->kp.SS <= 16 && nf >= 8192;
+    const bool streams = P == 1 && nf >= 65536 && nf <= 262144;
+    if (total <= 0xffffffffu && !light && !streams)
+        hipLaunchKernelGGL(fitness_kernel, dim3((unsigned)std::min<size_t>(nf, 1 << 20)), dim3(64), 0, s->stream,
+                           s->kp.storage, s->d_target, s->d_t2e, d_fit, threads, nf, P, s->kp.K, s->kp.SS,
+                           (int)f.experiments, (int)f.repetitions);
+    else
+        hipLaunchKernelGGL(fitness_each, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, s->stream, s->kp.storage,
+                           s->d_target, s->d_t2e, d_fit, threads, nf, P, s->kp.K, s->kp.SS, (int)f.experiments,
+                           (int)f.repetitions);
     HIPCHK(hipGetLastError(), "fitness_kernel launch");
     HIPCHK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
     HIPCHK(hipMemcpy(out, d_fit, sizeof(double) * nf, hipMemcpyDeviceToHost), "hipMemcpy D2H");
