@@ -828,11 +828,17 @@ void forward(ctl_mlp* n, int B, float* out, const float* t = nullptr, const int3
 }
 
 // Inference of B rows of x (device, FP32) into out: one fused launch for inner
-// widths up to 256 (four wavefronts of 64 columns), else layer by layer.
+// widths up to 256 (four wavefronts of 64 columns), else layer by layer.  A wide
+// output in few rows goes by layers too: the fused workgroups of 32 rows walk
+// its columns one after the other.  us of the call fused / by layers, 64, 2048
+// and 8192 rows: 1000 outputs behind 256s 37 / 35, 38 / 42, 44 / 63; 2000
+// behind 200 38 / 26, 40 / 38, 50 / 49; 3000 behind 200 47 / 25, 56 / 40, 63 /
+// 66; 8000 behind 256s 124 / 32, 125 / 53, 159 / 131.
 int infer(ctl_mlp* n, const float* x, int B, float* out) {
     int wmax = 0;
     for (int l = 0; l < n->L; ++l) wmax = std::max(wmax, n->widths[l]);
-    if (wmax <= 256 && n->L <= MLAYERS) {
+    const bool tall = n->widths[n->L] <= 1024 || B >= 8192;
+    if (wmax <= 256 && n->L <= MLAYERS && tall) {
         FusedArgs f{};
         f.x = x;
         f.y = out;

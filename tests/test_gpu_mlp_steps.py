@@ -87,3 +87,17 @@ def test_training_steps(ctl, gpu, widths, batch, cap):
         twin.close()
         p = got
     net.close()
+
+
+# outputs around 1024 and rows around 8192: fused or layer by layer, the same bits for the same row
+@pytest.mark.parametrize("widths", [[32, 200, 1024], [32, 200, 1025], [250, 256, 2100]])
+def test_inference_does_not_depend_on_the_rows_beside(ctl, gpu, widths):
+    print(f"case: mlp rows beside {widths}", flush=True)
+    net, p = _init(ctl, widths, seed=3)
+    x, _ = _data(widths, 8192, 4)
+    whole = net.forward(x)
+    for n in (1, 33, 500, 8191):
+        assert np.array_equal(net.forward(x[:n]), whole[:n]), n
+    want = om.forward(p, widths, x[:200], bf16=True)
+    assert np.linalg.norm(whole[:200] - want) <= FWD_REL * np.linalg.norm(want)
+    net.close()
