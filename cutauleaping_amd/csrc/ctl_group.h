@@ -1533,13 +1533,16 @@ __device__ __forceinline__ bool gregroup(int key, int reg, uint32_t* cnt, uint32
 // for four (128 VGPRs, a few bytes of scratch), measured +9 % at G = 16 and
 // +4 % at G = 32 on the 100x200 network, +24 % at G = 8 on the 50x100 sweep
 // network; G = 64 would spill heavily.  G = 2 and 4 hold three by themselves
-// except in mode 1 (174 VGPRs, where three waves have 168 each): two spilled
-// registers there give the third wave back (14 species and 40 reactions,
-// 262144 simulations, two / three: adaptive 35.6 / 26.4 ms, force-SSA
-// 29.6 / 21.0; larger models are bounded by LDS).  W > G serves runs that
-// leave the chip short of wavefronts.
-__host__ __device__ constexpr int gwaves(int G, int W, int PFM = 3) {
-    return W > G ? (W == 64 ? 2 : 4) : (G == 8 || G == 16 || G == 32 ? 4 : (G <= 4 && PFM == 1 ? 3 : 1));
+// except in mode 1 (174 VGPRs, where three waves have 168 each) and, with
+// regrouping, in mode 2 (170): up to two spilled registers there give the
+// third wave back (mode 1, 14 species and 40 reactions, 262144 simulations,
+// two / three: adaptive 35.6 / 26.4 ms, force-SSA 29.6 / 21.0; mode 2 with
+// regrouping every 8, 22 species and 24 reactions, G = 4: 8.4 / 6.5, 97 / 72;
+// larger models are bounded by LDS).  W > G serves runs that leave the chip
+// short of wavefronts.
+__host__ __device__ constexpr int gwaves(int G, int W, int PFM = 3, bool RG = false) {
+    const bool spill = PFM == 1 || (PFM == 2 && RG);
+    return W > G ? (W == 64 ? 2 : 4) : (G == 8 || G == 16 || G == 32 ? 4 : (G <= 4 && spill ? 3 : 1));
 }
 
 // Persistent group kernel: p.ns lanes = p.ns / W group slots, each pulling
@@ -1551,7 +1554,7 @@ __host__ __device__ constexpr int gwaves(int G, int W, int PFM = 3) {
 // running has switched, so that bursts run side by side.  Either way each simulation's events and draws are its own;
 // only the order in which the lanes serve the simulations moves.
 template <int G, int W, bool RG, int PF>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gwaves(G, W, PF)))) void group_kernel(KParams p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gwaves(G, W, PF, RG)))) void group_kernel(KParams p) {
     extern __shared__ uint32_t smem[];
     __shared__ float recip[64];
     __shared__ uint32_t rg_cnt[12];

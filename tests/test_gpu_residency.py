@@ -34,6 +34,20 @@ def test_a_full_chip_holds_three_wavefronts_a_simd(gpu, oracle_lib, S, R, order)
     m.close()
 
 
+@pytest.mark.parametrize("G,S,R,order", [(2, 22, 24, 1), (4, 22, 24, 3), (4, 13, 40, 1), (4, 22, 24, 1)])
+def test_regrouping_holds_three_wavefronts_a_simd(gpu, oracle_lib, G, S, R, order):
+    print(f"case: residency regrouping G={G} S={S} R={R} order={order}", flush=True)
+    left, right, c = _ring(S, R, order)
+    x0, ts = np.full((1, S), 30, np.uint32), np.array([0.01, 0.02])
+    m = gpu.Model.from_arrays(left, right, x0, c, ts)
+    with gpu.Sim(m, 131072, 1, seed=3, lanes_per_sim=G, compact_interval=8) as s:
+        s.run()
+        assert s.stats()["slots"] >= 196608
+        out, _ = oracle_lib.run(left, right, x0, c, ts, n=4096, seed=3, group=G, threads=8)
+        assert np.array_equal(s.samples()[:4096], out)
+    m.close()
+
+
 # more simulations than one instance's 64-lane teams hold, fewer than another's
 @pytest.mark.parametrize("S,R,order", [(22, 24, 3), (13, 40, 1), (22, 24, 1)])
 def test_widths_around_the_residency_bit_exact(gpu, oracle_lib, S, R, order):
