@@ -107,11 +107,11 @@ SIM_STAT_DTYPE = np.dtype([("firings", "u8"), ("ssa_steps", "u8"), ("poisson", "
 _lib = None
 
 
-def build(verbose: bool = False) -> None:
-    """Compiles libctl.so and the CLI for gfx950 (cutauleaping_amd/csrc/Makefile)."""
+def build(verbose: bool = False, force: bool = False) -> None:
+    """Compiles libctl.so and the CLI for gfx950 (cutauleaping_amd/csrc/Makefile); force: what is up to date too."""
     jobs = str(min(8, os.cpu_count() or 1))
     out = None if verbose else subprocess.DEVNULL
-    subprocess.run(["make", "-s", "-j", jobs, "-C", os.path.join(HERE, "csrc")], check=True,
+    subprocess.run(["make", "-s", "-j", jobs, "-C", os.path.join(HERE, "csrc")] + (["-B"] if force else []), check=True,
                    stdout=out)
 
 
